@@ -42,6 +42,7 @@ iteration i.
 
 from __future__ import annotations
 
+import weakref
 from collections.abc import Sequence
 from dataclasses import dataclass
 
@@ -91,12 +92,17 @@ class BatchExecutor:
                  use_graphs: bool = True) -> None:
         model.validate_storage(manager.storage)
         self.model = model
-        self.manager = manager
+        self._manager: PagedKVCacheManager | None = manager
+        self._manager_ref = weakref.ref(manager)
         self.builder = PackedBatchBuilder(manager.storage.device, manager.storage.block_size)
         graphs = DecodeGraphs(model, manager.storage)
         self.graphs = graphs if use_graphs and graphs.supported() else None
         self._token_host: list[torch.Tensor | None] = [None, None]
         self._token_turn = 0
+
+    @property
+    def manager(self) -> PagedKVCacheManager:
+        return self._manager_ref() if self._manager is None else self._manager
 
     def execute(self, prefill: Sequence[ScheduledRequest], decode: Sequence[ScheduledRequest],
                 *, metrics=None) -> tuple[str, ...]:
@@ -283,13 +289,15 @@ def _check_group(requests: Sequence[ScheduledRequest], kind: str) -> None:
 
 def _executor_for(model: LlamaModel, manager: PagedKVCacheManager) -> BatchExecutor:
     """The executor of (model, manager), so that callers looping over execute_decode
-    reuse its staging buffers and decode graphs. It is kept on the manager itself: the
-    two refer to each other, and the cycle (with the pools and graphs it holds) is
-    collected once the caller lets go of the manager."""
+    reuse its staging buffers and decode graphs. It is kept on the manager itself and
+    refers to it weakly: the pools and graphs go when the caller lets go of the manager,
+    and do not wait in a cycle for the collector (which may run while another graph is
+    captured, where freeing one is fatal)."""
 
     executor = getattr(manager, "_batch_executor", None)
     if executor is None or executor.model is not model:
         executor = BatchExecutor(model, manager)
+        executor._manager = None
         manager._batch_executor = executor
     return executor
 

@@ -31,6 +31,11 @@ after the metadata): the host then need not have read them back yet.
 
 from __future__ import annotations
 
+import gc
+import threading
+from collections.abc import Iterator
+from contextlib import contextmanager
+
 import numpy as np
 import torch
 
@@ -38,6 +43,29 @@ from tokserve_amd.batching.metadata import PackedBatch, SequenceWork
 from tokserve_amd.kernels import ops
 
 __all__ = ["DecodeGraphs"]
+
+_capturing = threading.Lock()
+
+
+@contextmanager
+def _uncollected() -> Iterator[None]:
+    """The cyclic collector held off while a stream captures.
+
+    A collection inside the capture may free another CUDAGraph (an engine's that became
+    garbage in a reference cycle), and torch's destructor of one synchronises the device.
+    That is refused while any stream captures, and an error in a destructor ends the
+    process. Collections due meanwhile run after the capture. The lock keeps two threads
+    from restoring the collector under each other's capture.
+    """
+
+    with _capturing:
+        enabled = gc.isenabled()
+        gc.disable()
+        try:
+            yield
+        finally:
+            if enabled:
+                gc.enable()
 
 
 class _Captured:
@@ -166,7 +194,7 @@ class DecodeGraphs:
         if len(self._graphs) < self.max_graphs:
             torch.cuda.synchronize(self.device)
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with _uncollected(), torch.cuda.graph(graph):
                 g_logits = self.model.forward_packed(batch, self.storage)
                 g_tokens = ops.greedy_argmax(g_logits).view(-1)
             self._graphs[key] = _Captured(graph, static, g_logits, g_tokens, {})
