@@ -1,35 +1,15 @@
-// Paged decode with MFMA scores, bf16/fp16, block size 16.
+// Paged decode on the matrix cores, bf16/fp16 queries, block size 16.
 //
-// Two kernels. decode_pv_kernel (further below) is the one every launch takes: both
-// products on the MFMA pipe, K/V pages HBM -> LDS by DMA. decode_mfma_kernel, the
-// earlier design described next, computes P.V on the VALU; it is compiled only with
-// kPvMfma set to false, to compare the two.
-//
-// decode_mfma_kernel: one workgroup of NW waves per (sequence, KV head[, split]). The pages of the
-// sequence are cut into NW contiguous ranges, one per wave; the waves' partial
-// softmax states (m, l, acc) are merged through LDS at the end, so no result
-// ever crosses workgroups inside the kernel (a cross-workgroup split, used only
-// for batches too small to fill the GPU, is merged by a second launch).
-//
-// Per page (16 x Dh contiguous elements of one KV head = one MFMA tile):
-//   S^T (16 rows x 16 tokens) = Q_rep . K^T   with v_mfma_f32_16x16x32_{bf16,f16}
-//     A operand: row m holds query head m % G of this KV group (replicated),
-//     B operand: column n holds token n of the page, straight from 16-byte
-//     HBM loads (lane (grp, r) reads dims c*32 + grp*8 .. +8 of token r);
-//     lane (grp, r) receives the scores of heads (grp*4 + i) % G for token r.
-// Softmax is online with a lazy reference: each lane checks its own scores
-// against reference + 8 (log2 units), and only when some score passes it does
-// the wave take row maxima, move the reference and rescale l and the P.V
-// accumulators (rare after a row's first page). The page's probabilities
-// (G x 16) go through a per-wave LDS slice. P.V runs on the VALU as packed
-// two-element dot products (v_dot2_f32_bf16 / _f16: P rounded to the model
-// dtype, V exact, fp32 accumulation): lane (hg, tg, dc) owns dims dc*8 .. +8
-// of heads hg*HPL .. +HPL and tokens tg*4 .. +3 of every page, so V also
-// arrives as 16-byte (fp8: 8-byte) loads, regrouped into token pairs by byte
-// permutes; the four token groups are summed once per wave. Every K/V byte is read from HBM exactly once
-// for all G query heads. Pages are double-buffered in registers and a wave's
-// block ids sit in one VGPR (broadcast with readlane), so nothing in the page
-// loop waits on a dependent memory access.
+// decode_pv_kernel: one workgroup of kWaves waves per (sequence, KV head[, split]). The
+// pages of the sequence (16 x Dh contiguous elements of one KV head) are cut into
+// kWaves contiguous ranges, one per wave; the waves' partial softmax states (m, l,
+// acc) are merged through LDS at the end, so no result ever crosses workgroups inside
+// the kernel (a cross-workgroup split, used only for batches too small to fill the
+// GPU, is merged by a second launch). Softmax is online with a lazy reference: each
+// lane checks its own scores against reference + 8 (log2 units), and only when some
+// score passes it does the wave take maxima, move the reference and rescale l and the
+// P.V accumulators (rare after a sequence's first page). Every K/V byte is read from
+// HBM exactly once for all G query heads.
 #include "attention_common.hpp"
 #include "rope_common.hpp"
 
@@ -37,26 +17,6 @@ namespace tks {
 namespace {
 
 constexpr int kWaves = 4;
-// s_waitcnt immediate: vmcnt 0, expcnt and lgkmcnt left at their maxima (no wait).
-constexpr int kWaitVmcntZero = 0x0F70;
-// Register pages per wave: the page being consumed and the next one in flight
-// (3 or 4 measured no faster, for bf16 and for fp8 pages, and cost occupancy).
-// (3 or 4 pages measured no faster at Dh 64 either, also at batches of two waves
-// per SIMD: there the page loop is bound by its own instruction latency.)
-constexpr int kRing = 2;
-
-template <int DH, int G>
-struct DecodeShape {
-  static constexpr int BS = 16;
-  static constexpr int NC = DH / 32;                // QK k-chunks of 32
-  static constexpr int LPR = DH / 8;                // lanes per V row (8 dims each)
-  static constexpr int TG = 4;                      // token groups (4 tokens each)
-  static constexpr int HG = 64 / (LPR * TG);        // head groups across the wave
-  static constexpr int HPL = G / HG;                // heads per lane in P.V
-  static_assert(DH == 64 || DH == 128, "head_dim");
-  static_assert(HG >= 1 && G % HG == 0 && 16 % G == 0, "group size");
-  static_assert(HPL * 8 <= 64, "P.V accumulator budget");
-};
 
 // Orders LDS traffic among the lanes of one wave (the waves of a workgroup run
 // different page counts, so a workgroup barrier cannot be used in the loop).
@@ -66,22 +26,14 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Packed pairs of the model dtype for the P.V dot products.
+// Two e4m3 codes of a word (bytes 0, 1, or 2, 3 with HI) as a pair of T, exactly.
 template <typename T>
-struct Dot2;
+struct Fp8Pair;
 template <>
-struct Dot2<bf16_t> {
+struct Fp8Pair<bf16_t> {
   typedef __bf16 pair __attribute__((ext_vector_type(2)));
-  static __device__ __forceinline__ float run(pair a, pair b, float c) {
-#if __HIP_DEVICE_COMPILE__
-    return __builtin_amdgcn_fdot2_f32_bf16(a, b, c, false);
-#else
-    return c;
-#endif
-  }
-  // Two e4m3 codes of a word (bytes 0, 1, or 2, 3 with HI) as a pair, exactly.
   template <bool HI>
-  static __device__ __forceinline__ pair from_fp8(uint32_t w) {
+  static __device__ __forceinline__ pair decode(uint32_t w) {
 #if __HIP_DEVICE_COMPILE__
     return __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI);
 #else
@@ -91,17 +43,10 @@ struct Dot2<bf16_t> {
   }
 };
 template <>
-struct Dot2<_Float16> {
+struct Fp8Pair<_Float16> {
   typedef _Float16 pair __attribute__((ext_vector_type(2)));
-  static __device__ __forceinline__ float run(pair a, pair b, float c) {
-#if __HIP_DEVICE_COMPILE__
-    return __builtin_amdgcn_fdot2(a, b, c, false);
-#else
-    return c;
-#endif
-  }
   template <bool HI>
-  static __device__ __forceinline__ pair from_fp8(uint32_t w) {
+  static __device__ __forceinline__ pair decode(uint32_t w) {
 #if __HIP_DEVICE_COMPILE__
     return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, HI);
 #else
@@ -111,96 +56,31 @@ struct Dot2<_Float16> {
   }
 };
 
-template <typename P>
-__device__ __forceinline__ P pair_bits(uint32_t w) {
-  P r;
-  __builtin_memcpy(&r, &w, 4);
-  return r;
-}
-
-// Byte permute: byte i of the result is byte sel_i of (hi : lo), bytes 0-3 from
-// lo and 4-7 from hi.
-__device__ __forceinline__ uint32_t byte_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
-#if __HIP_DEVICE_COMPILE__
-  return __builtin_amdgcn_perm(hi, lo, sel);
-#else
-  (void)hi, (void)sel;
-  return lo;
-#endif
-}
-
-// K/V rows as stored: T itself, or fp8 e4m3 decoded exactly to T (every e4m3
-// value is a bf16 and an f16), K as MFMA operands and V as token pairs for the
-// dot products. A lane's 8 elements of a row are one 16-byte load of T or one
-// 8-byte load of fp8.
+// Eight elements of a row as the pool stores them, T itself (16 bytes) or fp8 e4m3
+// (8 bytes, decoded exactly to T: every e4m3 value is a bf16 and an f16), and as an
+// MFMA operand.
 template <typename T, typename KV>
 struct PageIO {
   typedef uint4 raw;
-  typedef typename Dot2<T>::pair pair;
-  static __device__ __forceinline__ raw load(const KV *p) { return ld16_stream(p); }
   static __device__ __forceinline__ typename Mfma<T>::v8 k_operand(raw r) { return as_v8<T>(r); }
-  // Rows t0, t1 (8 elements each) as token pairs: vp[d] = {row t0[d], row t1[d]}.
-  static __device__ __forceinline__ void v_pairs(raw t0, raw t1, pair (&vp)[8]) {
-    const uint32_t a[4] = {t0.x, t0.y, t0.z, t0.w}, b[4] = {t1.x, t1.y, t1.z, t1.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      vp[2 * k] = pair_bits<pair>(byte_perm(b[k], a[k], 0x05040100u));
-      vp[2 * k + 1] = pair_bits<pair>(byte_perm(b[k], a[k], 0x07060302u));
-    }
-  }
-  static __device__ __forceinline__ raw zero() { return make_uint4(0, 0, 0, 0); }
 };
 template <typename T>
 struct PageIO<T, fp8e4m3_t> {
   typedef uint2 raw;
-  static __device__ __forceinline__ raw load(const fp8e4m3_t *p) {
-    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-    const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const u32x2 *>(p));
-    return make_uint2(v.x, v.y);
-  }
   static __device__ __forceinline__ typename Mfma<T>::v8 k_operand(raw r) {
     typename Mfma<T>::v8 o = {};
-#if __HIP_DEVICE_COMPILE__
     const uint32_t w[2] = {r.x, r.y};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      if constexpr (__is_same(T, bf16_t)) {
-        const auto lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.0f, false);
-        const auto hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.0f, true);
-        o[4 * i] = lo[0];
-        o[4 * i + 1] = lo[1];
-        o[4 * i + 2] = hi[0];
-        o[4 * i + 3] = hi[1];
-      } else {
-        const auto lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[i], 1.0f, false);
-        const auto hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[i], 1.0f, true);
-        o[4 * i] = lo[0];
-        o[4 * i + 1] = lo[1];
-        o[4 * i + 2] = hi[0];
-        o[4 * i + 3] = hi[1];
-      }
+      const auto lo = Fp8Pair<T>::template decode<false>(w[i]);
+      const auto hi = Fp8Pair<T>::template decode<true>(w[i]);
+      o[4 * i] = lo[0];
+      o[4 * i + 1] = lo[1];
+      o[4 * i + 2] = hi[0];
+      o[4 * i + 3] = hi[1];
     }
-#else
-    (void)r;
-#endif
     return o;
   }
-  typedef typename Dot2<T>::pair pair;
-  // Rows t0, t1 (8 e4m3 codes each) as token pairs of T, decoded exactly: the
-  // permutes put (t0[d], t1[d]) side by side, one conversion decodes a pair.
-  static __device__ __forceinline__ void v_pairs(raw t0, raw t1, pair (&vp)[8]) {
-    const uint32_t a[2] = {t0.x, t0.y}, b[2] = {t1.x, t1.y};
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const uint32_t x = byte_perm(b[k], a[k], 0x05010400u);  // t0.0 t1.0 t0.1 t1.1
-      const uint32_t y = byte_perm(b[k], a[k], 0x07030602u);  // t0.2 t1.2 t0.3 t1.3
-      vp[4 * k] = Dot2<T>::template from_fp8<false>(x);
-      vp[4 * k + 1] = Dot2<T>::template from_fp8<true>(x);
-      vp[4 * k + 2] = Dot2<T>::template from_fp8<false>(y);
-      vp[4 * k + 3] = Dot2<T>::template from_fp8<true>(y);
-    }
-  }
-  static __device__ __forceinline__ raw zero() { return make_uint2(0, 0); }
 };
 
 template <bool B>
@@ -349,382 +229,8 @@ __device__ __forceinline__ void write_staged_rows(const DecodeArgs &a, int b, in
   }
 }
 
-// ROPE: RoPE and the KV append of the sequence's new token fused in (DecodeArgs).
-// Every workgroup rotates its query rows as it loads them; the wave that reads the
-// sequence's last page stages the rotated key row and the value row in LDS, uses
-// them in place of what it loads of their slot and writes them to the pool after
-// its page loop, so no workgroup reads pool memory written in the same launch.
-// ROWS: fp8 pools with one scale per pool row (a.k_rs, a.v_rs); lane r of a page
-// loads its token's two scales with the page, multiplies its scores by the key
-// scale and its probabilities (after they enter the row sum) by the value scale.
-template <typename T, typename KV, int DH, int G, bool ROPE, bool ROWS = false>
-__global__ __launch_bounds__(64 * kWaves) void decode_mfma_kernel(DecodeArgs a) {
-  using S = DecodeShape<DH, G>;
-  constexpr int BS = S::BS, NC = S::NC, LPR = S::LPR, TG = S::TG, HPL = S::HPL;
-  using M = Mfma<T>;
-  using IO = PageIO<T, KV>;
-  using raw = typename IO::raw;
-  __shared__ __attribute__((aligned(16))) float p_s[kWaves][16][BS];  // rows >= G: padding
-  __shared__ __attribute__((aligned(16))) float alpha_s[kWaves][G];
-  __shared__ __attribute__((aligned(16))) float m_s[kWaves][G];
-  __shared__ __attribute__((aligned(16))) float l_s[kWaves][G];
-  __shared__ __attribute__((aligned(16))) float acc_s[kWaves][G][DH];
-  // The fused append's new key and value rows, in the pool's form, and the
-  // workgroup's G query rows (rotated when the RoPE is fused in).
-  __shared__ __attribute__((aligned(16))) KV new_k_s[ROPE ? DH : 1];
-  __shared__ __attribute__((aligned(16))) KV new_v_s[ROPE ? DH : 1];
-  __shared__ __attribute__((aligned(16))) T q_s[G * DH];
-
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 15;   // QK: token of the page
-  const int grp = lane >> 4; // QK: k-group / output row block
-  const int dc = lane % LPR;          // P.V: 8-dim chunk
-  const int tg = (lane / LPR) % TG;   // P.V: token group
-  const int hg = lane / (LPR * TG);   // P.V: head group
-
-  const int kvh = blockIdx.x;
-  const int split = blockIdx.z;
-  const int b = a.seq_order ? min(max(a.seq_order[blockIdx.y], 0), (int)gridDim.y - 1)
-                            : (int)blockIdx.y;
-  // A length above the host bound is clamped so no access can leave its buffer.
-  const int len = min(a.seq_lens[b], a.key_cap);
-  const int n_pages = (len + BS - 1) / BS;
-  const int p_begin = split * a.pages_per_split;
-  T *out = static_cast<T *>(a.out);
-  if (p_begin >= n_pages) {
-    if (split == 0) {  // empty sequence: defined all-zero output
-      for (int i = threadIdx.x; i < G * DH; i += 64 * kWaves)
-        out[b * a.o_ss + (int64_t)(kvh * G + i / DH) * a.o_hs + i % DH] = from_float<T>(0.f);
-      if constexpr (ROPE) {
-        if (n_pages == 0 && threadIdx.x < 64 &&
-            stage_new_rows<T, KV, DH, BS>(a, b, kvh, threadIdx.x, new_k_s, new_v_s)) {
-          wave_lds_sync();
-          write_staged_rows<T, KV, DH, BS>(a, b, kvh, threadIdx.x, new_k_s, new_v_s);
-        }
-      }
-    }
-    return;
-  }
-  const int p_end = min(n_pages, p_begin + a.pages_per_split);
-  const int per_wave = (p_end - p_begin + kWaves - 1) / kWaves;
-  const int w_begin = p_begin + wave * per_wave;
-  const int w_end = min(p_end, w_begin + per_wave);
-
-  // The QK dot product runs over the dims in any order Q and K share. Pools in
-  // the model dtype: MFMA c takes dims c*32 + grp*8 .. +8 (one 16-byte K load
-  // each). fp8 pools: lane group grp holds the contiguous slab of dims
-  // grp*NC*8 .. +NC*8 and MFMA c its c-th 8 dims, so a lane's K bytes of a page
-  // come in NC/2 16-byte loads instead of NC 8-byte ones.
-  constexpr bool kSlab = sizeof(KV) == 1;
-  typename M::v8 qa[NC];
-  // The workgroup's G query rows go through LDS once, a 16-byte chunk per thread
-  // (one rotation pair per thread when the RoPE is fused in), and every lane reads
-  // its MFMA chunks there: 1-2 % faster than each lane loading its chunks from global
-  // memory at small batches, and over e4m3 pools (slab layout, where a rotation
-  // pair's halves sit in different lane groups) the way to rotate without cross-lane
-  // moves. With the RoPE fused in, the wave whose range holds the sequence's last
-  // page stages the new rows in LDS first, so their loads overlap the barrier's wait;
-  // its lanes of the new token put them in place of what they load of that page, and
-  // after its page loop it writes them to the pool.
-  const int32_t *bt_row = a.bt + (int64_t)b * a.bt_stride;
-  bool staged = false;  // this wave staged the new rows (it writes them to the pool)
-  bool patch = false;   // ... and puts them in place of its loads (length not clamped)
-  const int new_off = ROPE ? (len - 1) % BS : 0;
-  {
-    const int t = threadIdx.x;
-    if constexpr (ROPE) {
-      constexpr int HALF = DH / 2;
-      if (w_begin < w_end && w_end == n_pages) {  // wave-uniform
-        staged = stage_new_rows<T, KV, DH, BS>(a, b, kvh, lane, new_k_s, new_v_s);
-        patch = staged && a.seq_lens[b] == len;
-        wave_lds_sync();
-      }
-      if (t < G * HALF / 8) {
-        const int64_t pos = min(max(a.positions[b], (int64_t)0), a.table_len - 1);
-        const int h = t / (HALF / 8), j = (t % (HALF / 8)) * 8;
-        const T *qrow =
-            static_cast<const T *>(a.q) + b * a.q_ss + (int64_t)(kvh * G + h) * a.q_hs;
-        float cf[8], sf[8], o1[8], o2[8];
-        load_table<T, 8>(static_cast<const T *>(a.cos_t) + pos * HALF,
-                         static_cast<const T *>(a.sin_t) + pos * HALF, j, cf, sf);
-        rotate_values<T, 8>(qrow + j, cf, sf, HALF, o1, o2);
-        st16(&q_s[h * DH + j], pack<T>(o1));
-        st16(&q_s[h * DH + j + HALF], pack<T>(o2));
-      }
-    } else {
-      if (t < G * DH / 8) {
-        const int h = t / (DH / 8), j = (t % (DH / 8)) * 8;
-        const T *qrow =
-            static_cast<const T *>(a.q) + b * a.q_ss + (int64_t)(kvh * G + h) * a.q_hs;
-        st16(&q_s[h * DH + j], ld16(qrow + j));
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-      qa[c] = as_v8<T>(ld16(&q_s[(r % G) * DH + (kSlab ? grp * NC * 8 + c * 8 : c * 32 + grp * 8)]));
-  }
-
-  const KV *kc = static_cast<const KV *>(a.kc) + a.pool.layer_base + (int64_t)kvh * a.pool.head_stride;
-  const KV *vc = static_cast<const KV *>(a.vc) + a.pool.layer_base + (int64_t)kvh * a.pool.head_stride;
-  const int k_off = r * DH + grp * (kSlab ? NC * 8 : 8);
-  const int v_off = tg * 4 * DH + dc * 8;
-
-  float acc[HPL][8];
-#pragma unroll
-  for (int j = 0; j < HPL; ++j)
-#pragma unroll
-    for (int d = 0; d < 8; ++d) acc[j][d] = 0.f;
-  // Per row i of this lane (head (grp*4 + i) % G, token r): m = reference max
-  // in log2 units (-inf before the first key), l = this lane's share of the sum;
-  // thr = m + 8 (a score above it moves the reference) and mref = the value
-  // subtracted before exp2 (m, or 0 while m is -inf), both updated only when
-  // the reference moves.
-  float m[4], l[4], thr[4], mref[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
-    thr[i] = -INFINITY;
-    mref[i] = 0.f;
-  }
-  const float scale_log2 = a.scale_log2;
-
-  // Row scales of token r of a page: ks_row[blk * rows_per_block].
-  const int64_t rows_per_block = a.pool.block_stride / DH;
-  const float *ks_row = nullptr;
-  const float *vs_row = nullptr;
-  if constexpr (ROWS) {
-    const int64_t base = (a.pool.layer_base + (int64_t)kvh * a.pool.head_stride) / DH + r;
-    ks_row = a.k_rs + base;
-    vs_row = a.v_rs + base;
-  }
-  // Every page is read once: non-temporal loads.
-  auto load_page = [&](int blk_reg, int idx, raw (&kr)[NC], raw (&vr)[4], float &ks, float &vs) {
-    const int64_t blk = clamp_block(__builtin_amdgcn_readlane(blk_reg, idx), a.pool.num_blocks);
-    if constexpr (ROWS) {
-      ks = ks_row[blk * rows_per_block];
-      vs = vs_row[blk * rows_per_block];
-    }
-    const KV *kp = kc + blk * a.pool.block_stride + k_off;
-    const KV *vp = vc + blk * a.pool.block_stride + v_off;
-    if constexpr (kSlab) {
-      static_assert(NC % 2 == 0, "fp8 K slab in 16-byte loads");
-#pragma unroll
-      for (int c = 0; c < NC; c += 2) {
-        const uint4 u = ld16_stream(kp + c * 8);
-        kr[c] = raw{u.x, u.y};
-        kr[c + 1] = raw{u.z, u.w};
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < NC; ++c) kr[c] = IO::load(kp + c * 32);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) vr[j] = IO::load(vp + j * DH);
-  };
-
-  using pair = typename IO::pair;
-  // vr is the ring's page: rows past the sequence's last key are zeroed in place
-  // (the slot is reloaded before its next use). Only a wave's last page can be
-  // the sequence's last page, so the page loop's steady state passes
-  // kCheckEnd = false and skips the check; its drain passes true.
-  // The fused append's new rows in place of what was loaded of the sequence's last
-  // page (only a wave's last page can be it: the page loop's drain).
-  auto substitute_new_rows = [&](raw (&kr)[NC], raw (&vr)[4], int p) {
-    if (patch && p == n_pages - 1) {
-      if (r == new_off) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-          kr[c] = load_chunk<T, KV>(new_k_s + (kSlab ? grp * NC * 8 + c * 8 : c * 32 + grp * 8));
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (tg * 4 + j == new_off) vr[j] = load_chunk<T, KV>(new_v_s + dc * 8);
-    }
-  };
-  auto consume = [&](auto check_end, const raw (&kr)[NC], raw (&vr)[4], int p, float ks,
-                     float vs) {
-    constexpr bool kCheckEnd = decltype(check_end)::value;
-    typename M::f4 s4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < NC; ++c) s4 = M::run(qa[c], IO::k_operand(kr[c]), s4);
-    float sv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sv[i] = s4[i] * scale_log2;
-    if constexpr (ROWS) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sv[i] *= ks;
-    }
-    // The sequence's last page (uniform): keys past len score -inf, and their V
-    // rows, whatever the pool holds there, are zeroed, since 0 * NaN is NaN.
-    if (kCheckEnd && (p + 1) * BS > len) {
-      const bool valid = p * BS + r < len;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sv[i] = valid ? sv[i] : -INFINITY;
-      if constexpr (ROWS) vs = valid ? vs : 0.f;  // an unwritten row's scale may be NaN
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (p * BS + tg * 4 + j >= len) vr[j] = IO::zero();
-    }
-    bool over = false;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) over = over || sv[i] > thr[i];
-    // A score more than 8 above its row's reference (every row on the first
-    // page): row maxima, new references, l rescaled here and the P.V
-    // accumulators below (alpha through LDS).
-    const bool rebase = __builtin_amdgcn_ballot_w64(over) != 0;
-    if (rebase) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float mx = row16_max(sv[i]);
-        const bool bump = mx > thr[i];
-        const float alpha = bump ? fast_exp2(m[i] - mx) : 1.f;
-        m[i] = bump ? mx : m[i];
-        thr[i] = m[i] + 8.f;
-        mref[i] = m[i] == -INFINITY ? 0.f : m[i];
-        l[i] *= alpha;
-        const int h = grp * 4 + i;
-        if (h < G && r == 0) alpha_s[wave][h] = alpha;
-      }
-    }
-    // Rows past G (lane groups replicating heads) land in padding rows of p_s.
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float pv = fast_exp2(sv[i] - mref[i]);
-      l[i] += pv;
-      p_s[wave][grp * 4 + i][r] = ROWS ? pv * vs : pv;
-    }
-    wave_lds_sync();
-    pair vp[2][8];
-    IO::v_pairs(vr[0], vr[1], vp[0]);
-    IO::v_pairs(vr[2], vr[3], vp[1]);
-#pragma unroll
-    for (int j = 0; j < HPL; ++j) {
-      const int h = hg * HPL + j;
-      if (rebase) {
-        const float al = alpha_s[wave][h];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) acc[j][d] *= al;
-      }
-      const float4 pv = *reinterpret_cast<const float4 *>(&p_s[wave][h][tg * 4]);
-      pair p01, p23;
-      p01[0] = static_cast<typename M::elem>(pv.x);
-      p01[1] = static_cast<typename M::elem>(pv.y);
-      p23[0] = static_cast<typename M::elem>(pv.z);
-      p23[1] = static_cast<typename M::elem>(pv.w);
-#pragma unroll
-      for (int d = 0; d < 8; ++d)
-        acc[j][d] = Dot2<T>::run(vp[1][d], p23, Dot2<T>::run(vp[0][d], p01, acc[j][d]));
-    }
-    wave_lds_sync();
-  };
-
-  // A ring of kRing register pages: the steady-state loop always has the next
-  // kRing - 1 pages' loads issued behind the page being consumed (straight-line,
-  // so the wait before each consume covers only its own page); the last pages
-  // of a 64-page chunk drain in the epilogue.
-  constexpr int D = kRing;
-  for (int c0 = w_begin; c0 < w_end; c0 += 64) {
-    const int n = min(w_end, c0 + 64) - c0;
-    const int blk_reg = lane < n ? bt_row[c0 + lane] : 0;
-    // Wait for the block ids here, while no page load is in flight (the previous
-    // chunk's ring has drained). Without this the compiler, which cannot place this
-    // load in the page loop's count of outstanding loads, waits for every load in
-    // flight at each loop iteration before it reads a block id, and the register
-    // ring never holds more than the one page being consumed.
-    __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
-    raw kb[D][NC], vb[D][4];
-    float ksr[D] = {}, vsr[D] = {};
-#pragma unroll
-    for (int j = 0; j < D - 1; ++j)
-      if (j < n) load_page(blk_reg, j, kb[j], vb[j], ksr[j], vsr[j]);
-    int i = 0;  // page i sits in ring slot i % D
-    for (; i + 2 * D - 1 <= n; i += D) {
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        load_page(blk_reg, i + j + D - 1, kb[(j + D - 1) % D], vb[(j + D - 1) % D],
-                  ksr[(j + D - 1) % D], vsr[(j + D - 1) % D]);
-        consume(BoolConst<false>{}, kb[j], vb[j], c0 + i + j, ksr[j], vsr[j]);
-      }
-    }
-    // Fewer than 2D - 1 pages left; those before i + D - 1 are already loaded.
-#pragma unroll
-    for (int j = 0; j < 2 * D - 2; ++j) {
-      if (i + j < n) {
-        if (i + j + D - 1 < n)
-          load_page(blk_reg, i + j + D - 1, kb[(j + D - 1) % D], vb[(j + D - 1) % D],
-                    ksr[(j + D - 1) % D], vsr[(j + D - 1) % D]);
-        if constexpr (ROPE) substitute_new_rows(kb[j % D], vb[j % D], c0 + i + j);
-        consume(BoolConst<true>{}, kb[j % D], vb[j % D], c0 + i + j, ksr[j % D], vsr[j % D]);
-      }
-    }
-  }
-
-  // The staged rows to the pool, once this wave has read the page that holds their slot.
-  if constexpr (ROPE) {
-    if (staged) write_staged_rows<T, KV, DH, BS>(a, b, kvh, lane, new_k_s, new_v_s);
-  }
-
-  // Per-wave state: l summed over the 16 tokens, acc over the 4 token groups.
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    l[i] = row16_sum(l[i]);
-    const int h = grp * 4 + i;
-    if (h < G && r == 0) {
-      m_s[wave][h] = m[i];
-      l_s[wave][h] = l[i];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < HPL; ++j)
-#pragma unroll
-    for (int d = 0; d < 8; ++d) {
-      acc[j][d] += __shfl_xor(acc[j][d], LPR, 64);
-      acc[j][d] += __shfl_xor(acc[j][d], 2 * LPR, 64);
-    }
-  if (tg == 0) {
-#pragma unroll
-    for (int j = 0; j < HPL; ++j) {
-      float *dst = &acc_s[wave][hg * HPL + j][dc * 8];
-      *reinterpret_cast<float4 *>(dst) = make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
-      *reinterpret_cast<float4 *>(dst + 4) =
-          make_float4(acc[j][4], acc[j][5], acc[j][6], acc[j][7]);
-    }
-  }
-  __syncthreads();
-
-  // Merge the waves (a wave without pages has m = -inf, l = 0, acc = 0).
-  const bool single = a.max_splits == 1;
-  for (int i = threadIdx.x; i < G * DH; i += 64 * kWaves) {
-    const int h = i / DH, d = i % DH;
-    float M_ = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) M_ = fmaxf(M_, m_s[w][h]);
-    float L = 0.f, o = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const float e = m_s[w][h] == -INFINITY ? 0.f : fast_exp2(m_s[w][h] - M_);
-      L += e * l_s[w][h];
-      o += e * acc_s[w][h][d];
-    }
-    // v_scale (1 for pools in the model dtype, an exact no-op) decodes V.
-    if (single) {
-      out[b * a.o_ss + (int64_t)(kvh * G + h) * a.o_hs + d] = from_float<T>(o / L * a.v_scale);
-    } else {
-      const int64_t w = ((int64_t)b * a.num_q_heads + kvh * G + h) * a.max_splits + split;
-      if (d == 0) {
-        a.ws_m[w] = M_;
-        a.ws_l[w] = L;
-      }
-      a.ws_acc[w * DH + d] = o * a.v_scale;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// P.V on the matrix cores, for pools in the model dtype (bf16 / fp16).
+// The page step: both products on the MFMA pipe, K/V pages HBM -> LDS by DMA.
 //
 // Per page the score MFMA runs with its operands swapped: S (16 tokens x 16 head
 // columns) = K . Q^T with v_mfma_f32_16x16x32 (A = the page's K rows, B = Q^T,
@@ -764,8 +270,8 @@ __device__ __forceinline__ void decode_fp8_chunk(u32x4 w, u32x4 &lo, u32x4 &hi) 
   uint32_t o[8];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const auto p0 = Dot2<T>::template from_fp8<false>(w[k]);
-    const auto p1 = Dot2<T>::template from_fp8<true>(w[k]);
+    const auto p0 = Fp8Pair<T>::template decode<false>(w[k]);
+    const auto p1 = Fp8Pair<T>::template decode<true>(w[k]);
     __builtin_memcpy(&o[2 * k], &p0, 4);
     __builtin_memcpy(&o[2 * k + 1], &p1, 4);
   }
@@ -1185,8 +691,8 @@ void decode_pv_kernel(DecodeArgs a) {
   const int w_begin = p_begin + wave * per_wave;
   const int w_end = min(p_end, w_begin + per_wave);
 
-  // Q^T operands through LDS as in decode_mfma_kernel (rotated there when the RoPE
-  // is fused in; the wave holding the sequence's last page stages the new rows).
+  // Q^T operands through LDS (rotated there when the RoPE is fused in; the wave
+  // holding the sequence's last page stages the new rows).
   typename M::v8 qa[NC];
   const int32_t *bt_row = a.bt + (int64_t)b * a.bt_stride;
   bool staged = false;
@@ -1477,7 +983,7 @@ void decode_pv_kernel(DecodeArgs a) {
         for (int t = 0; t < DT; ++t) {
           uint32_t nv;
           if constexpr (kFp8) {
-            const auto pr = Dot2<T>::template from_fp8<false>(lds_read1_now(new_v_s + t * 16 + r));
+            const auto pr = Fp8Pair<T>::template decode<false>(lds_read1_now(new_v_s + t * 16 + r));
             uint32_t both;
             __builtin_memcpy(&both, &pr, 4);
             nv = both & 0xFFFFu;
@@ -1588,9 +1094,6 @@ void decode_pv_kernel(DecodeArgs a) {
   }
 }
 
-// Pools in the model dtype take the P.V-on-MFMA kernel.
-constexpr bool kPvMfma = true;
-
 template <typename T, typename KV, bool ROPE = false>
 int32_t launch_typed(const DecodeArgs &a, int32_t num_seqs, int32_t num_kv_heads, int32_t G,
                      int32_t head_dim, hipStream_t s) {
@@ -1601,18 +1104,11 @@ int32_t launch_typed(const DecodeArgs &a, int32_t num_seqs, int32_t num_kv_heads
   if (head_dim == DH && G == GG) {                                                  \
     if constexpr (sizeof(KV) == 1) {                                                \
       if (a.k_rs != nullptr) {                                                      \
-        if constexpr (kPvMfma || ROPE)                                              \
-          decode_pv_kernel<T, KV, DH, GG, ROPE, true><<<grid, 64 * kWaves, 0, s>>>(a); \
-        else                                                                        \
-          decode_mfma_kernel<T, KV, DH, GG, false, true><<<grid, 64 * kWaves, 0, s>>>(a); \
+        decode_pv_kernel<T, KV, DH, GG, ROPE, true><<<grid, 64 * kWaves, 0, s>>>(a); \
         return check_launch();                                                      \
       }                                                                             \
     }                                                                               \
-    if constexpr (kPvMfma) {                                                        \
-      decode_pv_kernel<T, KV, DH, GG, ROPE><<<grid, 64 * kWaves, 0, s>>>(a);        \
-    } else {                                                                        \
-      decode_mfma_kernel<T, KV, DH, GG, ROPE><<<grid, 64 * kWaves, 0, s>>>(a);      \
-    }                                                                               \
+    decode_pv_kernel<T, KV, DH, GG, ROPE><<<grid, 64 * kWaves, 0, s>>>(a);          \
     return check_launch();                                                          \
   }
   TKS_DECODE(128, 4)
