@@ -189,6 +189,13 @@ struct Mfma<_Float16> {
   }
 };
 
+// D (16 x 16) += A (16 x 4) . B (4 x 16) in fp32: lane (g, r) holds A[r][g] and B[g][r], and
+// D[4 g + i][r].
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
 template <typename T>
 __device__ __forceinline__ typename Mfma<T>::v8 as_v8(uint4 v) {
   typename Mfma<T>::v8 r;
@@ -214,7 +221,7 @@ struct DecodeArgs {
   const int32_t *seq_order;  // workgroup z -> sequence (null: identity)
   int32_t num_q_heads;
   float scale_log2;
-  int32_t pages_per_split;
+  int32_t pages_per_split;  // 16-token pages (block_pages to a block)
   int32_t max_splits;
   int32_t key_cap;  // keys any sequence may have: min(table width, splits * split size) * BS
   void *out;
@@ -235,6 +242,7 @@ struct DecodeArgs {
   int64_t kn_ss = 0, kn_hs = 0, vn_ss = 0, vn_hs = 0;
   const int64_t *slots = nullptr;
   float k_scale = 1.f;  // e4m3 pools: the new key row is stored as e4m3(key / k_scale)
+  int32_t block_pages = 1;  // 16-token pages to a block
 };
 
 // fp8 pools with one fp32 scale per pool row (token, KV head): the row's scale is
@@ -295,15 +303,21 @@ int32_t launch_prefill_mfma(const PrefillArgs &a, int32_t dtype, int32_t num_seq
                             int32_t num_kv_heads, int32_t group, int32_t head_dim,
                             int32_t max_query_len, hipStream_t stream);
 
-// Shapes the MFMA decode kernel is instantiated for (block size 16).
-bool decode_mfma_supported(int32_t dtype, int32_t head_dim, int32_t group);
+// Shapes the MFMA decode kernel is instantiated for: block sizes that are multiples of
+// 16, pools whose page ids fit 32 bits.
+bool decode_mfma_supported(int32_t dtype, int32_t head_dim, int32_t group, int32_t block_size,
+                           int64_t num_blocks, int32_t num_kv_heads);
 
 // Launches the MFMA decode kernel over grid (max_splits, Hkv, B); returns a tks_status.
 // With max_splits == 1 it writes the output, otherwise split partials to be merged.
 // fp8_pools: K/V pools hold e4m3 (DecodeArgs.scale_log2 then carries k_scale,
-// DecodeArgs.v_scale the V factor).
+// DecodeArgs.v_scale the V factor). launch_decode_blocks: its part for blocks of more
+// than one page.
 int32_t launch_decode_mfma(const DecodeArgs &a, int32_t dtype, int32_t num_seqs,
                            int32_t num_kv_heads, int32_t group, int32_t head_dim,
                            hipStream_t stream, bool fp8_pools);
+int32_t launch_decode_blocks(const DecodeArgs &a, int32_t dtype, int32_t num_seqs,
+                             int32_t num_kv_heads, int32_t group, int32_t head_dim,
+                             hipStream_t stream, bool fp8_pools);
 
 }  // namespace tks

@@ -7,7 +7,7 @@
 // online in fp32 (:125-136) and the output is acc / sum in the query dtype (:138).
 //
 // Decode (one query per sequence) goes to decode_pv_kernel (decode_mfma.hip)
-// for bf16/fp16 with block size 16 and Dh 64/128; every other shape and fp32
+// for bf16/fp16 with block sizes that are multiples of 16 and Dh 64/128; every other shape and fp32
 // (where 1e-5 parity wants fp32 products) uses attn_generic_kernel below:
 // one 4-wave workgroup per (query row, KV head, split), 64 keys per wave step
 // on the VALU. The
@@ -395,42 +395,47 @@ __global__ __launch_bounds__(128) void merge_splits_kernel(
 // ------------------------------------------------------------------------
 
 // Key splits for decode. A (sequence, KV head) pair runs as one workgroup
-// whose four waves walk its pages in order, so an unsplit launch lasts at least
+// whose four waves walk its keys in order, so an unsplit launch lasts at least
 // as long as its longest sequence takes; with few pairs that chain, not the
-// bytes, sets the time. Splits are merged by a second launch.
+// bytes, sets the time. Splits are merged by a second launch. The lengths below are in
+// keys: of blocks that are multiples of 16, so that their size does not change the
+// split; for other block sizes a block counts as 16 (`unit` = block_size).
 //  * Fewer than kFillItems pairs (less than one workgroup per CU): cut every
-//    sequence so the batch has about kFillItems workgroups, splits of 16 to 48
-//    pages (fp32 decode step, 8 sequences x 2 KV heads, contexts <= 513: 12.8 +
+//    sequence so the batch has about kFillItems workgroups, splits of 256 to 768
+//    keys (fp32 decode step, 8 sequences x 2 KV heads, contexts <= 513: 12.8 +
 //    4.0 us merge split against 18.4 us unsplit; 8 / 16 Llama-3-8B sequences x 8
-//    KV heads, contexts log-uniform in [128, 8192]: 39.3 / 41.8 us at 64 pages,
-//    34.8 / 37.0 us at 48, 39.3 / 45.9 us at 16; 16 sequences unsplit: 59 us).
-//  * Fewer than kSplitBelowItems pairs and a length bound of kSplitFromPages
-//    pages or more: 32-page splits (32 / 64 such Llama-3-8B sequences with the
-//    MFMA P.V kernel, split and merge: 45.3 / 90.5 us at 32 pages, 47.6 / 91.2 at
-//    64, 74.1 / 110.7 unsplit).
+//    KV heads, contexts log-uniform in [128, 8192]: 39.3 / 41.8 us at 1,024 keys,
+//    34.8 / 37.0 us at 768, 39.3 / 45.9 us at 256; 16 sequences unsplit: 59 us).
+//  * Fewer than kSplitBelowItems pairs and a length bound of kSplitFromKeys or
+//    more: 512-key splits (32 / 64 such Llama-3-8B sequences with the
+//    MFMA P.V kernel, split and merge: 45.3 / 90.5 us at 512 keys, 47.6 / 91.2 at
+//    1,024, 74.1 / 110.7 unsplit).
 //  * Otherwise unsplit: 128, 192 and 256 Llama-3-8B sequences (128: 161.4 us
-//    against 166.2 at 64 pages and 173.3 at 32; 192: 216.4 against 249.6+ split),
+//    against 166.2 at 1,024 keys and 173.3 at 512; 192: 216.4 against 249.6+ split),
 //    and short contexts (128 sequences x 4 KV heads, Dh 64, contexts up to 1152
 //    under a 2048-token bound).
 constexpr int64_t kFillItems = 256;
-constexpr int64_t kMinSplitPages = 16;
-constexpr int64_t kMaxFillSplitPages = 48;
+constexpr int64_t kMinSplitUnits = 16;
+constexpr int64_t kMaxFillSplitUnits = 48;
 constexpr int64_t kSplitBelowItems = 1024;
-constexpr int64_t kSplitPages = 32;
-constexpr int64_t kSplitFromPages = 256;
+constexpr int64_t kSplitUnits = 32;
+constexpr int64_t kSplitFromUnits = 256;
+
+int32_t split_unit(int32_t block_size) { return block_size % 16 == 0 ? 16 : block_size; }
 
 int32_t choose_pages_per_split(int32_t num_seqs, int32_t num_kv_heads, int32_t block_size,
-                               int32_t max_seq_len, int32_t requested) {
+                               int32_t max_seq_len, int32_t requested, int32_t unit) {
   if (requested > 0) return requested;
   const int64_t max_pages = ceil_div(max_seq_len > 0 ? max_seq_len : 1, block_size);
   const int64_t items = static_cast<int64_t>(num_seqs) * num_kv_heads;
+  int64_t keys = max_pages * block_size;
   if (items > 0 && items < kFillItems) {
-    const int64_t per_split = ceil_div(max_pages, ceil_div(kFillItems, items));
-    return static_cast<int32_t>(std::min(kMaxFillSplitPages, std::max(kMinSplitPages, per_split)));
+    const int64_t per_split = ceil_div(max_pages, ceil_div(kFillItems, items)) * block_size;
+    keys = std::min(kMaxFillSplitUnits * unit, std::max(kMinSplitUnits * unit, per_split));
+  } else if (items < kSplitBelowItems && keys >= kSplitFromUnits * unit) {
+    keys = kSplitUnits * unit;
   }
-  if (items < kSplitBelowItems && max_pages >= kSplitFromPages)
-    return static_cast<int32_t>(kSplitPages);
-  return static_cast<int32_t>(max_pages);
+  return static_cast<int32_t>(ceil_div(keys, block_size));
 }
 
 int32_t split_count(int32_t max_seq_len, int32_t block_size, int32_t pps) {
@@ -504,10 +509,11 @@ int32_t vec_rows_ok(const void *kc, const void *vc, int32_t head_dim, int elem) 
   return aligned16(kc) && aligned16(vc) && (head_dim * elem) % 16 == 0;
 }
 
-bool mfma_eligible(int32_t dtype, int32_t block_size, int32_t head_dim, int32_t G,
-                   const void *q, int64_t q_ss, int64_t q_hs, const void *kc, const void *vc,
+bool mfma_eligible(int32_t dtype, int64_t num_blocks, int32_t num_kv_heads, int32_t block_size,
+                   int32_t head_dim, int32_t G, const void *q, int64_t q_ss, int64_t q_hs, const void *kc, const void *vc,
                    const void *out, int64_t o_ss, int64_t o_hs) {
-  if (block_size != 16 || !decode_mfma_supported(dtype, head_dim, G)) return false;
+  if (!decode_mfma_supported(dtype, head_dim, G, block_size, num_blocks, num_kv_heads))
+    return false;
   return aligned16(q) && aligned16(kc) && aligned16(vc) && aligned16(out) && q_ss % 8 == 0 &&
          q_hs % 8 == 0 && o_ss % 8 == 0 && o_hs % 8 == 0;
 }
@@ -528,7 +534,8 @@ extern "C" int64_t tks_paged_attention_decode_workspace_bytes(int32_t num_seqs,
       block_size <= 0 || max_seq_len < 0 || pages_per_split < 0)
     return -1;
   const int32_t pps =
-      choose_pages_per_split(num_seqs, num_kv_heads, block_size, max_seq_len, pages_per_split);
+      choose_pages_per_split(num_seqs, num_kv_heads, block_size, max_seq_len, pages_per_split,
+                             split_unit(block_size));
   const int32_t max_splits = split_count(max_seq_len, block_size, pps);
   if (max_splits <= 1) return 0;
   return carve(nullptr, num_seqs, num_q_heads, max_splits, head_dim).bytes;
@@ -577,7 +584,8 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
     return TKS_ERR_VALUE;
 
   const int32_t pps =
-      choose_pages_per_split(num_seqs, num_kv_heads, block_size, max_seq_len, pages_per_split);
+      choose_pages_per_split(num_seqs, num_kv_heads, block_size, max_seq_len, pages_per_split,
+                             split_unit(block_size));
   const int32_t max_splits = split_count(max_seq_len, block_size, pps);
   if (max_splits > kMaxGridSplits) return TKS_ERR_VALUE;
   Workspace w = carve(workspace, num_seqs, num_q_heads, max_splits, head_dim);
@@ -590,9 +598,9 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float scale_log2 = scale * kLog2e * k_scale;
 
-  const bool mfma = mfma_eligible(dtype, block_size, head_dim, G, query, q_seq_stride,
-                                  q_head_stride, key_cache, value_cache, out, out_seq_stride,
-                                  out_head_stride);
+  const bool mfma = mfma_eligible(dtype, num_blocks, num_kv_heads, block_size, head_dim, G, query,
+                                  q_seq_stride, q_head_stride, key_cache, value_cache, out,
+                                  out_seq_stride, out_head_stride);
   if (ra != nullptr) {
     // Fused when the MFMA kernel runs with its new rows in 16-byte chunks; otherwise
     // the RoPE + append launch writes the rotated queries into `out`, which the
@@ -645,6 +653,9 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
                  v_scale};
     a.k_rs = k_rs;
     a.v_rs = v_rs;
+    a.block_pages = block_size / 16;
+    a.pages_per_split = static_cast<int32_t>(
+        std::min<int64_t>(static_cast<int64_t>(pps) * a.block_pages, INT32_MAX));
     if (ra != nullptr) {
       a.positions = ra->positions;
       a.cos_t = ra->cos_cache;
@@ -825,9 +836,18 @@ extern "C" int32_t tks_paged_attention_decode_noalloc(
     int32_t num_seqs, int32_t num_q_heads, int32_t max_seq_len, float scale,
     int32_t pages_per_split, void *out, int64_t out_seq_stride, int64_t out_head_stride,
     int32_t dtype, tks_stream_t stream) {
-  const int64_t needed = tks_paged_attention_decode_workspace_bytes(
+  int64_t needed = tks_paged_attention_decode_workspace_bytes(
       num_seqs, num_q_heads, num_kv_heads, head_dim, block_size, max_seq_len, pages_per_split);
   if (needed < 0) return TKS_ERR_VALUE;
+  if (needed > kStaticScratchBytes && pages_per_split == 0 && split_unit(block_size) < block_size) {
+    // Long blocks: splits of as many blocks as a batch over blocks of 16 has, i.e.
+    // fewer and longer ones, before the batch is refused.
+    pages_per_split = choose_pages_per_split(num_seqs, num_kv_heads, block_size, max_seq_len, 0,
+                                             block_size);
+    needed = tks_paged_attention_decode_workspace_bytes(num_seqs, num_q_heads, num_kv_heads,
+                                                        head_dim, block_size, max_seq_len,
+                                                        pages_per_split);
+  }
   if (needed > kStaticScratchBytes) return TKS_ERR_WORKSPACE;
   void *ws = nullptr;
   if (needed > 0) {
