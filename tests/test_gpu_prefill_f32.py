@@ -1,0 +1,103 @@
+"""fp32 prefill on the matrix cores against the oracle in 64 bits.
+
+rtol 1e-5, atol 1e-6 as for every fp32 result (the parity contract); outputs here average
+values of unit size, and each is a handful of chains of at most a few hundred fp32 sums.
+"""
+
+import pytest
+import torch
+from torch.testing import assert_close
+
+from oracle import paged
+from tokserve_amd import workloads
+from tokserve_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+
+TOL = dict(rtol=1e-5, atol=1e-6)
+POOL_SCALES = dict(k_scale=0.5, v_scale=0.25)
+
+
+def _run(batch, keys, values, **scales):
+    out = ops.paged_attention_prefill(
+        batch.query, keys, values, batch.block_tables, batch.seq_lens, batch.cu_seqlens_q,
+        layer_index=0, max_query_len=batch.max_query_len, max_seq_len=batch.max_seq_len, **scales)
+    torch.cuda.synchronize()
+    return out.cpu()
+
+
+def _oracle(batch, keys, values):
+    return paged.prefill_batch(batch.query.cpu(), keys, values, batch.block_tables.cpu(),
+                               batch.seq_lens.cpu(), batch.cu_seqlens_q.cpu(), 0, torch.float64)
+
+
+# Contexts and chunks around a step's 32 keys, a page and a tile of 128 / G query tokens.
+CONTEXTS, CHUNKS = [1, 32, 33, 64, 65, 200, 300, 77], [1, 32, 33, 17, 64, 129, 1, 16]
+
+
+@pytest.mark.parametrize("pool", ["same", "fp8", "fp8_rows"])
+@pytest.mark.parametrize(("hq", "hkv", "dh", "block_size"),
+                         [(32, 4, 64, 16), (8, 2, 128, 32), (2, 2, 128, 16), (16, 1, 64, 16),
+                          (6, 2, 64, 7), (5, 1, 128, 48)])
+def test_prefill_f32_shapes(device, hq, hkv, dh, block_size, pool) -> None:
+    batch = workloads.paged_batch(CONTEXTS, CHUNKS, num_q_heads=hq, num_kv_heads=hkv, head_dim=dh,
+                                  block_size=block_size, dtype=torch.float32, device=device,
+                                  seed=dh + hq)
+    keys, values = batch.key_cache.cpu(), batch.value_cache.cpu()
+    if pool == "same":
+        got = _run(batch, batch.key_cache, batch.value_cache)
+    elif pool == "fp8":
+        k8 = paged.quantize_e4m3(keys, POOL_SCALES["k_scale"])
+        v8 = paged.quantize_e4m3(values, POOL_SCALES["v_scale"])
+        got = _run(batch, k8.to(device), v8.to(device), **POOL_SCALES)
+        keys = paged.dequantize_e4m3(k8, POOL_SCALES["k_scale"], torch.float32)
+        values = paged.dequantize_e4m3(v8, POOL_SCALES["v_scale"], torch.float32)
+    else:
+        (k8, ks), (v8, vs) = paged.quantize_e4m3_rows(keys), paged.quantize_e4m3_rows(values)
+        got = _run(batch, k8.to(device), v8.to(device), k_scales=ks.to(device),
+                   v_scales=vs.to(device))
+        keys = paged.dequantize_e4m3_rows(k8, ks, torch.float64)
+        values = paged.dequantize_e4m3_rows(v8, vs, torch.float64)
+    assert_close(got, _oracle(batch, keys, values), **TOL)
+
+
+def test_prefill_f32_strided_rows_and_moving_reference(device) -> None:
+    """Query and output rows inside wider ones, and keys that grow along each sequence, so
+    that the softmax reference moves many times."""
+
+    batch = workloads.paged_batch([700, 40], [200, 40], num_q_heads=8, num_kv_heads=2,
+                                  head_dim=64, block_size=16, dtype=torch.float32, device=device,
+                                  seed=3)
+    for b, context in enumerate([700, 40]):
+        for i in range((context + 15) // 16):
+            batch.key_cache[0, int(batch.block_tables[b, i])] *= 1 + i / 8
+    wide = torch.zeros(240, 8, 72, device=device)
+    wide[..., :64] = batch.query
+    out = torch.full((240, 12, 64), 7.0, device=device)
+    ops.paged_attention_prefill(
+        wide[..., :64], batch.key_cache, batch.value_cache, batch.block_tables, batch.seq_lens,
+        batch.cu_seqlens_q, layer_index=0, max_query_len=200, max_seq_len=700, out=out[:, :8])
+    torch.cuda.synchronize()
+    expected = _oracle(batch, batch.key_cache.cpu(), batch.value_cache.cpu())
+    # Scores reach ~30 here, where one fp32 rounding is up to 2^-20; a sum of Dh products
+    # gathers about sqrt(Dh) = 8 of them, so an exponent is off by up to 8e-6 and an output
+    # by twice that times the largest |v| (~4).
+    assert_close(out[:, :8].cpu(), expected, rtol=0, atol=6e-5)
+    assert bool((out[:, 8:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dh", [64, 128])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_prefill_f32_values_past_a_row_do_not_reach_it(device, dh, bad) -> None:
+    """A value that is not finite reaches the rows that see its key and no other."""
+
+    batch = workloads.paged_batch([100, 90], [60, 90], num_q_heads=4, num_kv_heads=1, head_dim=dh,
+                                  block_size=16, dtype=torch.float32, device=device, seed=5)
+    clean = _oracle(batch, batch.key_cache.cpu(), batch.value_cache.cpu())
+    key = 70  # query token 30 of the first chunk
+    batch.value_cache[0, int(batch.block_tables[0, key // 16]), 0, key % 16, dh - 3] = bad
+    got = _run(batch, batch.key_cache, batch.value_cache)
+    hit = torch.zeros_like(got, dtype=torch.bool)
+    hit[30:60, :, dh - 3] = True
+    assert not bool(got[hit].isfinite().any())
+    assert_close(got[~hit], clean[~hit], **TOL)

@@ -287,7 +287,62 @@ struct PrefillArgs {
   float v_scale = 1.f;  // V decode factor (pages decoded from fp8 pools; 1 otherwise)
   const int32_t *seq_order = nullptr;  // rank -> sequence (null: identity)
   int32_t num_seqs = 0;
+  // fp8 pools with one scale per pool row (launch_prefill_f32; null: per-pool scales).
+  const float *k_rs = nullptr, *v_rs = nullptr;
 };
+
+// Query tiles (QT tokens of one sequence) of a prefill batch of up to 64 sequences, by the
+// keys they need, most first: tile i of that order. Lane b of the wave looks at sequence b;
+// a tile's level is its keys in units of QT, rounded up, and a search over the levels (at
+// most max_level) finds the one item i falls in, so no workgroup is launched for a tile
+// that does not exist and none of the longest is started last. Every wave finds the same
+// (about 9 rounds of a wave sum); false past the last tile.
+constexpr int kTileOrderSeqs = 64;
+struct QueryTile {
+  int seq, tile;
+};
+__device__ __forceinline__ int wave_sum_int(int x) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+  return x;
+}
+__device__ __forceinline__ bool find_query_tile(const int32_t *cu_q, const int32_t *seq_lens,
+                                                int num_seqs, int QT, int max_level, int i,
+                                                int lane, QueryTile *out) {
+  int q_len = 0, base = 0;
+  if (lane < num_seqs) {
+    q_len = max(0, cu_q[lane + 1] - cu_q[lane]);
+    base = seq_lens[lane] - q_len;
+  }
+  const int tiles = (q_len + QT - 1) / QT;
+  const int first = base >= 0 ? (base + QT - 1) / QT : -((-base) / QT);  // ceil(base / QT)
+  // Tiles of this lane's sequence at level k or above: those that end past (k - 1) QT keys.
+  auto above = [&](int k) {
+    if (k > max_level) return 0;
+    if (k <= 0) return tiles;
+    if (base + q_len <= (k - 1) * QT) return 0;
+    return tiles - min(tiles, max(0, k - 1 - first));
+  };
+  if (i >= wave_sum_int(tiles)) return false;
+  int lo = 0, hi = max_level + 1;  // total(lo) > i >= total(hi)
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (wave_sum_int(above(mid)) > i) lo = mid; else hi = mid;
+  }
+  const int rem = i - wave_sum_int(above(lo + 1));
+  const int mine = above(lo) - above(lo + 1);
+  int before = mine;  // inclusive sum over the lanes, then exclusive
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(before, o, 64);
+    if (lane >= o) before += x;
+  }
+  before -= mine;
+  const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(rem >= before && rem < before + mine));
+  out->seq = at;
+  out->tile = __shfl(tiles - above(lo) + rem - before, at, 64);
+  return true;
+}
 
 // 16-key pages of one sequence the MFMA prefill kernel holds in LDS: it serves
 // sequences of up to kPrefillBtWindow * 16 keys.
@@ -302,6 +357,13 @@ bool prefill_mfma_supported(int32_t dtype, int32_t head_dim, int32_t group, int3
 int32_t launch_prefill_mfma(const PrefillArgs &a, int32_t dtype, int32_t num_seqs,
                             int32_t num_kv_heads, int32_t group, int32_t head_dim,
                             int32_t max_query_len, hipStream_t stream);
+
+// The fp32 prefill on the matrix cores (16-byte aligned rows, scale_log2 > 0), over fp32
+// or e4m3 pools; returns a tks_status.
+bool prefill_f32_supported(int32_t head_dim, int32_t group);
+int32_t launch_prefill_f32(const PrefillArgs &a, int32_t num_seqs, int64_t num_tokens,
+                           int32_t num_kv_heads, int32_t group, int32_t head_dim,
+                           int32_t max_query_len, bool fp8_pools, hipStream_t stream);
 
 // Shapes the MFMA decode kernel is instantiated for: block sizes that are multiples of
 // 16, pools whose page ids fit 32 bits.

@@ -10,9 +10,9 @@
 // for bf16/fp16 with block sizes that are multiples of 16 and Dh 64/128; every other shape and fp32
 // (where 1e-5 parity wants fp32 products) uses attn_generic_kernel below:
 // one 4-wave workgroup per (query row, KV head, split), 64 keys per wave step
-// on the VALU. The
-// generic kernel is also the ragged chunked-prefill path (one row per query
-// token, causal key length).
+// on the VALU. Prefill goes to prefill_mfma.hip (bf16/fp16) and prefill_f32.hip; the
+// generic kernel takes the chunks neither supports (one row per query token, causal
+// key length).
 //
 // A decode batch with fewer (sequence, KV head) pairs than it takes to fill the
 // GPU is also split across workgroups along the keys; the split partials
@@ -781,6 +781,23 @@ int32_t prefill_impl(const void *query, int64_t q_token_stride, int64_t q_head_s
     return launch_prefill_mfma(p, dtype, num_seqs, num_kv_heads, G, head_dim, max_query_len, s);
   }
   const int kv_elem = fp8_pools ? 1 : elem_bytes(dtype);
+  // fp32 queries: fp32 products on the matrix cores (16 prompts of 64 to 1,024 tokens,
+  // 32 / 4 heads, Dh 64: 828 us on the VALU kernel below, 124 us). Row maxima of raw
+  // scores again need a positive scale.
+  if (dtype == TKS_FLOAT32 && scale_log2 > 0.f && scale_log2 < INFINITY &&
+      prefill_f32_supported(head_dim, G) && aligned16(query) && aligned16(out) &&
+      aligned16(key_cache) && aligned16(value_cache) && q_token_stride % 4 == 0 &&
+      q_head_stride % 4 == 0 && out_token_stride % 4 == 0 && out_head_stride % 4 == 0) {
+    PrefillArgs p{query,    q_token_stride, q_head_stride, key_cache,    value_cache,
+                  pool,     block_tables,   block_table_stride, seq_lens, cu_seqlens_q,
+                  scale_log2, key_cap,      out,           out_token_stride, out_head_stride};
+    p.v_scale = v_scale;
+    p.seq_order = seq_order;
+    p.k_rs = k_rs;
+    p.v_rs = v_rs;
+    return launch_prefill_f32(p, num_seqs, num_tokens, num_kv_heads, G, head_dim, max_query_len,
+                              fp8_pools, s);
+  }
   GenericArgs a{query,     q_token_stride, q_head_stride, key_cache,  value_cache, pool,
                 block_tables, block_table_stride, seq_lens, nullptr, cu_seqlens_q, num_seqs, num_q_heads,
                 G,         scale_log2,     pps,           1,          key_cap,     out,         out_token_stride,
