@@ -370,6 +370,14 @@ int32_t launch_prefill_f32(const PrefillArgs &a, int32_t num_seqs, int64_t num_t
 bool decode_mfma_supported(int32_t dtype, int32_t head_dim, int32_t group, int32_t block_size,
                            int64_t num_blocks, int32_t num_kv_heads);
 
+// fp32 decode on the matrix cores (decode_f32.hip), 16-byte aligned rows; `wide`: 8
+// waves per workgroup instead of 4. The RoPE and append are fused over fp32 pools only.
+bool decode_f32_supported(int32_t head_dim, int32_t group, int32_t block_size, int64_t num_blocks,
+                          int32_t num_kv_heads);
+int32_t launch_decode_f32(const DecodeArgs &a, int32_t num_seqs, int32_t num_kv_heads,
+                          int32_t group, int32_t head_dim, bool wide, bool fp8_pools,
+                          hipStream_t stream);
+
 // Launches the MFMA decode kernel over grid (max_splits, Hkv, B); returns a tks_status.
 // With max_splits == 1 it writes the output, otherwise split partials to be merged.
 // fp8_pools: K/V pools hold e4m3 (DecodeArgs.scale_log2 then carries k_scale,

@@ -7,8 +7,8 @@
 // online in fp32 (:125-136) and the output is acc / sum in the query dtype (:138).
 //
 // Decode (one query per sequence) goes to decode_pv_kernel (decode_mfma.hip)
-// for bf16/fp16 with block sizes that are multiples of 16 and Dh 64/128; every other shape and fp32
-// (where 1e-5 parity wants fp32 products) uses attn_generic_kernel below:
+// for bf16/fp16 and to decode_f32_kernel (decode_f32.hip) for fp32, both with block sizes
+// that are multiples of 16 and Dh 64/128; every other shape uses attn_generic_kernel below:
 // one 4-wave workgroup per (query row, KV head, split), 64 keys per wave step
 // on the VALU. Prefill goes to prefill_mfma.hip (bf16/fp16) and prefill_f32.hip; the
 // generic kernel takes the chunks neither supports (one row per query token, causal
@@ -402,8 +402,7 @@ __global__ __launch_bounds__(128) void merge_splits_kernel(
 // split; for other block sizes a block counts as 16 (`unit` = block_size).
 //  * Fewer than kFillItems pairs (less than one workgroup per CU): cut every
 //    sequence so the batch has about kFillItems workgroups, splits of 256 to 768
-//    keys (fp32 decode step, 8 sequences x 2 KV heads, contexts <= 513: 12.8 +
-//    4.0 us merge split against 18.4 us unsplit; 8 / 16 Llama-3-8B sequences x 8
+//    keys (8 / 16 Llama-3-8B sequences x 8
 //    KV heads, contexts log-uniform in [128, 8192]: 39.3 / 41.8 us at 1,024 keys,
 //    34.8 / 37.0 us at 768, 39.3 / 45.9 us at 256; 16 sequences unsplit: 59 us).
 //  * Fewer than kSplitBelowItems pairs and a length bound of kSplitFromKeys or
@@ -420,6 +419,7 @@ constexpr int64_t kMaxFillSplitUnits = 48;
 constexpr int64_t kSplitBelowItems = 1024;
 constexpr int64_t kSplitUnits = 32;
 constexpr int64_t kSplitFromUnits = 256;
+constexpr int32_t kWideKeys = 640;  // fp32: see decode_impl
 
 int32_t split_unit(int32_t block_size) { return block_size % 16 == 0 ? 16 : block_size; }
 
@@ -601,14 +601,21 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
   const bool mfma = mfma_eligible(dtype, num_blocks, num_kv_heads, block_size, head_dim, G, query,
                                   q_seq_stride, q_head_stride, key_cache, value_cache, out,
                                   out_seq_stride, out_head_stride);
+  const bool f32 = dtype == TKS_FLOAT32 &&
+                   decode_f32_supported(head_dim, G, block_size, num_blocks, num_kv_heads) &&
+                   aligned16(query) && aligned16(key_cache) && aligned16(value_cache) &&
+                   aligned16(out) && q_seq_stride % 4 == 0 && q_head_stride % 4 == 0 &&
+                   out_seq_stride % 4 == 0 && out_head_stride % 4 == 0;
   if (ra != nullptr) {
-    // Fused when the MFMA kernel runs with its new rows in 16-byte chunks; otherwise
-    // the RoPE + append launch writes the rotated queries into `out`, which the
+    // Fused when an MFMA kernel runs with its new rows in 16-byte chunks (fp32: over fp32
+    // pools); otherwise the RoPE + append launch writes the rotated queries into `out`, which the
     // decode then reads as its query (each workgroup reads its rows before it, or
     // the merge, writes them).
-    const bool fused = mfma && aligned16(ra->key) && aligned16(ra->value) &&
-                       aligned16(ra->cos_cache) && aligned16(ra->sin_cache) && ra->k_ss % 8 == 0 && ra->k_hs % 8 == 0 &&
-                       ra->v_ss % 8 == 0 && ra->v_hs % 8 == 0;
+    const int chunk = f32 ? 4 : 8;
+    const bool fused = (mfma || (f32 && !fp8_pools)) && aligned16(ra->key) &&
+                       aligned16(ra->value) && aligned16(ra->cos_cache) &&
+                       aligned16(ra->sin_cache) && ra->k_ss % chunk == 0 &&
+                       ra->k_hs % chunk == 0 && ra->v_ss % chunk == 0 && ra->v_hs % chunk == 0;
     if (!fused) {
       void *kc = const_cast<void *>(key_cache), *vc = const_cast<void *>(value_cache);
       const int32_t st0 =
@@ -645,10 +652,17 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
   }
 
   int32_t st;
-  if (mfma) {
+  // A small fp32 batch of short sequences runs unsplit, with more waves per workgroup, and
+  // saves the merge launch. One CU then does a pair's products, so only while they are
+  // short: 8 sequences x 2 KV heads, Dh 64, cold: 14 us up to 513 keys and 19.5 us up to
+  // 1,024, against 9.6 us and a merge of 4.7 us.
+  const bool wide = f32 && pages_per_split == 0 && max_splits > 1 && max_seq_len <= kWideKeys &&
+                    static_cast<int64_t>(num_seqs) * num_kv_heads < kFillItems;
+  const int32_t splits = wide ? 1 : max_splits;
+  if (mfma || f32) {
     DecodeArgs a{query,      q_seq_stride, q_head_stride, key_cache,   value_cache,
                  pool,       block_tables, block_table_stride, seq_lens, seq_order, num_q_heads,
-                 scale_log2, pps,          max_splits,    key_cap,     out,
+                 scale_log2, pps,          splits,        key_cap,     out,
                  out_seq_stride, out_head_stride, w.m,    w.l,         w.acc,
                  v_scale};
     a.k_rs = k_rs;
@@ -656,6 +670,7 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
     a.block_pages = block_size / 16;
     a.pages_per_split = static_cast<int32_t>(
         std::min<int64_t>(static_cast<int64_t>(pps) * a.block_pages, INT32_MAX));
+    if (wide) a.pages_per_split = key_cap / 16;
     if (ra != nullptr) {
       a.positions = ra->positions;
       a.cos_t = ra->cos_cache;
@@ -670,7 +685,8 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
       a.slots = ra->slot_mapping;
       a.k_scale = k_scale;
     }
-    st = launch_decode_mfma(a, dtype, num_seqs, num_kv_heads, G, head_dim, s, fp8_pools);
+    st = f32 ? launch_decode_f32(a, num_seqs, num_kv_heads, G, head_dim, wide, fp8_pools, s)
+             : launch_decode_mfma(a, dtype, num_seqs, num_kv_heads, G, head_dim, s, fp8_pools);
   } else {
     const int kv_elem = fp8_pools ? 1 : elem_bytes(dtype);
     GenericArgs a{query,     q_seq_stride, q_head_stride, key_cache, value_cache, pool,
@@ -682,7 +698,7 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
     a.v_rs = v_rs;
     st = launch_generic(a, dtype, num_seqs, num_kv_heads, fp8_pools, s);
   }
-  if (st != TKS_OK || max_splits == 1) return st;
+  if (st != TKS_OK || splits == 1) return st;
   const dim3 grid(num_q_heads, num_seqs);
   const int threads = head_dim > 64 ? 128 : 64;  // one thread per output element
 #define TKS_MERGE(TYPE)                                                                         \
