@@ -302,9 +302,12 @@ struct QueryTile {
   int seq, tile;
 };
 __device__ __forceinline__ int wave_sum_int(int x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
+  x += __builtin_amdgcn_mov_dpp(x, kDppQuadSwap1, 0xF, 0xF, true);
+  x += __builtin_amdgcn_mov_dpp(x, kDppQuadSwap2, 0xF, 0xF, true);
+  x += __builtin_amdgcn_mov_dpp(x, kDppHalfMirror, 0xF, 0xF, true);
+  x += __builtin_amdgcn_mov_dpp(x, kDppMirror, 0xF, 0xF, true);
+  return (__builtin_amdgcn_readlane(x, 0) + __builtin_amdgcn_readlane(x, 16)) +
+         (__builtin_amdgcn_readlane(x, 32) + __builtin_amdgcn_readlane(x, 48));
 }
 __device__ __forceinline__ bool find_query_tile(const int32_t *cu_q, const int32_t *seq_lens,
                                                 int num_seqs, int QT, int max_level, int i,
@@ -355,7 +358,7 @@ bool prefill_mfma_supported(int32_t dtype, int32_t head_dim, int32_t group, int3
 
 // Launches the MFMA prefill kernel over grid (query tiles, Hkv, B); returns a tks_status.
 int32_t launch_prefill_mfma(const PrefillArgs &a, int32_t dtype, int32_t num_seqs,
-                            int32_t num_kv_heads, int32_t group, int32_t head_dim,
+                            int64_t num_tokens, int32_t num_kv_heads, int32_t group, int32_t head_dim,
                             int32_t max_query_len, hipStream_t stream);
 
 // The fp32 prefill on the matrix cores (16-byte aligned rows, scale_log2 > 0), over fp32

@@ -764,7 +764,8 @@ int32_t prefill_impl(const void *query, int64_t q_token_stride, int64_t q_head_s
                   scale_log2, key_cap,      out,           out_token_stride, out_head_stride};
     p.seq_order = seq_order;
     p.num_seqs = num_seqs;
-    return launch_prefill_mfma(p, dtype, num_seqs, num_kv_heads, G, head_dim, max_query_len, s);
+    return launch_prefill_mfma(p, dtype, num_seqs, num_tokens, num_kv_heads, G, head_dim,
+                               max_query_len, s);
   }
   if (mfma_shape) {
     // fp8 pools: decode the batch's pages into the scratch pool, then the MFMA
@@ -794,7 +795,8 @@ int32_t prefill_impl(const void *query, int64_t q_token_stride, int64_t q_head_s
     p.v_scale = v_scale;
     p.seq_order = seq_order;
     p.num_seqs = num_seqs;
-    return launch_prefill_mfma(p, dtype, num_seqs, num_kv_heads, G, head_dim, max_query_len, s);
+    return launch_prefill_mfma(p, dtype, num_seqs, num_tokens, num_kv_heads, G, head_dim,
+                               max_query_len, s);
   }
   const int kv_elem = fp8_pools ? 1 : elem_bytes(dtype);
   // fp32 queries: fp32 products on the matrix cores (16 prompts of 64 to 1,024 tokens,

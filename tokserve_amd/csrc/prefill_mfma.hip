@@ -1,9 +1,9 @@
 // Chunked-prefill paged attention with MFMA for both products, bf16/fp16, block
 // sizes that are multiples of 16 (keys move in 16-key pages).
 //
-// One workgroup (4 waves) per (sequence, KV head, tile of QT query tokens). The
-// tile's rows are (token, query head) pairs, row = token * G + head, 128 rows
-// per workgroup, RT 16-row tiles per wave. Keys are processed 32 at a time
+// One workgroup (4 waves, or two groups of 4) per (sequence, KV head, tile of QT query
+// tokens). The tile's rows are (token, query head) pairs, row = token * G + head, 128 rows
+// (64 in batches of few tiles), RT 16-row tiles per wave. Keys are processed 32 at a time
 // (two pages). Per step every wave computes, per 16-row tile,
 //
 //   S^T (32 keys x 16 rows) = K . Q^T          2 x (Dh/32) v_mfma_f32_16x16x32
@@ -32,6 +32,8 @@
 // The causal mask is key <= query position, query i of sequence b sitting at
 // seq_lens[b] - q_len_b + i (tokserve/kernels/_triton_paged_attention.py:118-123).
 #include "attention_common.hpp"
+
+#include <algorithm>
 
 namespace tks {
 namespace {
@@ -223,8 +225,12 @@ struct Swizzle {
 template <int DH>
 constexpr int kPrefillOccupancy = DH == 64 ? 4 : 2;
 
-template <typename T, int DH, int G, int RT>
-__global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
+// NG = 2 splits a tile's steps between two groups of kPWaves waves (even and odd steps),
+// each with its own ring and sums, merged through LDS at the end: batches with fewer tiles
+// than CUs can hold last as long as their longest tile's chain of steps, which this halves
+// (launch_typed's rule).
+template <typename T, int DH, int G, int RT, int NG>
+__global__ __launch_bounds__(64 * kPWaves * NG) __attribute__((amdgpu_waves_per_eu(
     kPrefillOccupancy<DH>, kPrefillOccupancy<DH>))) void prefill_mfma_kernel(PrefillArgs a) {
   constexpr int ROWS = kPWaves * RT * 16;
   constexpr int QT = ROWS / G;           // query tokens per workgroup
@@ -246,11 +252,14 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
   typedef typename M::f4 f4;
   typedef typename M::v8 v8;
 
-  __shared__ __attribute__((aligned(16))) T ring[kStages * STAGE];
-  __shared__ int32_t bt_s[kPrefillBtWindow];
+  __shared__ __attribute__((aligned(16))) T rings[NG * kStages * STAGE];
+  __shared__ __attribute__((aligned(16))) int32_t bt_s[kPrefillBtWindow];
 
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = NG == 1 ? wave_all : wave_all % kPWaves;
+  const int grp = NG == 1 ? 0 : wave_all / kPWaves;
+  T *ring = rings + grp * (kStages * STAGE);
   const int lane = tid & 63;
   const int r = lane & 15;
   const int g = lane >> 4;
@@ -279,7 +288,8 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
   // Keys needed by the last token of the tile (causal); the host keeps key_cap
   // within the LDS block-id window.
   const int n_keys = max(0, min(min(kv_len, base_pos + t_end), kPrefillBtWindow * 16));
-  const int n_steps = (n_keys + KS - 1) / KS;
+  // Steps per group, the same for both: group 1's last may lie past the keys (all masked).
+  const int n_steps = (n_keys + NG * KS - 1) / (NG * KS);
   const int n_pages = (n_keys + 15) / 16;
 
   const T *q = static_cast<const T *>(a.q);
@@ -298,7 +308,7 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
 
   // Page units of the sequence (pages of the last step past the keys map to
   // unit 0: loaded, never used).
-  for (int i = tid; i < n_steps * (KS / 16); i += 64 * kPWaves)
+  for (int i = tid; i < n_steps * NG * (KS / 16); i += 64 * kPWaves * NG)
     bt_s[i] = i < n_pages ? (int32_t)clamp_block(bt_row[i / ppb], a.pool.num_blocks) * units_per_block + i % ppb
                           : 0;
 
@@ -331,7 +341,7 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
   // Load k of wave w fills 16-byte slots (k*kPWaves + w)*64 + lane of a tile;
   // slot = row * CPR + physical chunk. All rows of one load lie in one page.
   auto page_of_load = [&](int step, int k) {
-    return step * (KS / 16) + ((k * kPWaves + wave) * 64 / CPR) / 16;
+    return (step * NG + grp) * (KS / 16) + ((k * kPWaves + wave) * 64 / CPR) / 16;
   };
   using Swz = Swizzle<DH>;
   // Byte offsets of this lane's K and V chunks inside their page: LDS slot
@@ -483,7 +493,7 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
     for (int d = 0; d < DT; ++d) o[j][d] *= alpha;
   };
 
-  // One step: keys s*KS .. s*KS + KS - 1 from ring stage STG, whose K operands
+  // One step: keys k0 .. k0 + KS - 1, the group's s-th, from ring stage STG, whose K operands
   // are already in kraw. Pipeline: V(s) LDS reads overlap QK(s) and the
   // softmax; tile 1's QK MFMAs run under tile 0's softmax and tile 0's PV MFMAs
   // under tile 1's probabilities; then K(s+1) is read. With one barrier per
@@ -496,15 +506,16 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
   // mask work.
   int32_t blk_pair[LOADS];  // block ids of step s+3, read in the pair's first step s-1
   auto step = [&](auto stage_c, int s) {
-    static_assert(RT == 2, "the step interleaves two row tiles");
+    static_assert(RT == 1 || RT == 2, "the step interleaves two row tiles, or takes one");
     constexpr int STG = decltype(stage_c)::value;
     constexpr int O0 = STG * kStageBytes;
     constexpr int N0 = ((STG + 1) % kStages) * kStageBytes;
     // Block ids of the step whose loads this step hands to issue().
     const int ahead = min(s + (kPairs ? 4 : 3), n_steps - 1);
     const uint32_t ba = bt_base + page_of_load(ahead, 0) * 4;
-    const bool tail = s * KS + KS > n_keys;
-    const bool need_mask = s * KS + KS - 1 > min_pos || tail;
+    const int k0 = (s * NG + grp) * KS;
+    const bool tail = k0 + KS > n_keys;
+    const bool need_mask = k0 + KS - 1 > min_pos || tail;
     u32x2 vraw[2 * DT];
     uint32_t bid[LOADS];
     Reads::template values<O0, O0 + kRowsBytes>(va_addr, ba, vraw, bid);
@@ -513,10 +524,10 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
     k_operands(ka);
     f4 st[RT][2];
     scores(ka, 0, st[0]);
-    // Key kp = s*KS + kt*16 + g*4 + i is visible to a row iff kp <= qpos
+    // Key kp = k0 + kt*16 + g*4 + i is visible to a row iff kp <= qpos
     // (which also keeps it below n_keys).
     auto mask = [&](int j) {
-      const int rel = qpos[j] - (s * KS + g * 4);
+      const int rel = qpos[j] - (k0 + g * 4);
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -526,26 +537,31 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
     v8 pb[RT];
     float ps[RT];
     if (need_mask) mask(0);
-    scores(ka, 1, st[1]);
+    if constexpr (RT == 2) scores(ka, 1, st[1]);
     const float lm0 = lane_max(st[0]);
     bool over = lm0 > thr[0];
     ps[0] = probs(st[0], negref[0], pb[0]);
     // Tile 0's probabilities issue between tile 1's QK MFMAs (one MFMA, then
     // three VALU instructions), and stay here rather than sinking past the
     // rebase branch below.
+    if constexpr (RT == 2) {
 #pragma unroll
-    for (int i = 0; i < 2 * NC; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+      for (int i = 0; i < 2 * NC; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+      }
     }
     pin_vgpr(pb[0]);
     pin_vgpr(ps[0]);
-    if (need_mask) mask(1);
-    const float lm1 = lane_max(st[1]);
-    over = over || lm1 > thr[1];
+    float lm1 = 0.f;
+    if constexpr (RT == 2) {
+      if (need_mask) mask(1);
+      lm1 = lane_max(st[1]);
+      over = over || lm1 > thr[1];
+    }
     if (__builtin_amdgcn_ballot_w64(over)) {
       rebase(0, lm0);
-      rebase(1, lm1);
+      if constexpr (RT == 2) rebase(1, lm1);
       ps[0] = probs(st[0], negref[0], pb[0]);
     }
 
@@ -561,23 +577,25 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
       // probabilities are 0, and 0 * NaN would not be.
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int key = s * KS + (e / 4) * 16 + g * 4 + (e % 4);
+        const int key = k0 + (e / 4) * 16 + g * 4 + (e % 4);
         if (key >= n_keys) {
 #pragma unroll
           for (int d = 0; d < DT; ++d) va[d][e] = static_cast<typename M::elem>(0.f);
         }
       }
     }
-    ps[1] = probs(st[1], negref[1], pb[1]);
+    if constexpr (RT == 2) ps[1] = probs(st[1], negref[1], pb[1]);
 #pragma unroll
     for (int j = 0; j < RT; ++j)
 #pragma unroll
       for (int d = 0; d < DT; ++d) o[j][d] = M::run(va[d], pb[j], o[j][d]);
     // Tile 1's probabilities issue between tile 0's PV MFMAs.
+    if constexpr (RT == 2) {
 #pragma unroll
-    for (int d = 0; d < DT; ++d) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+      for (int d = 0; d < DT; ++d) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+      }
     }
 
     if (s + 1 < n_steps) {
@@ -630,6 +648,44 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
     }
   }
 
+  if constexpr (NG == 2) {
+    // Group 1's sums to the lanes of group 0 that hold the same rows and dims, through the
+    // rings' memory once every wave is done with it.
+    constexpr int kSums = RT * DT;
+    static_assert(kSums * kPWaves * 64 * 16 <= NG * kStages * STAGE * (int)sizeof(T), "merge area");
+    static_assert(2 * RT * kPWaves * 64 <= kPrefillBtWindow, "merge state");
+    float4 *o_s = reinterpret_cast<float4 *>(rings) + wave * 64 + lane;
+    float *st_s = reinterpret_cast<float *>(bt_s) + wave * 64 + lane;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (grp == 1) {
+#pragma unroll
+      for (int j = 0; j < RT; ++j) {
+        st_s[(2 * j) * kPWaves * 64] = thr[j] == -INFINITY ? -INFINITY : -negref[j];
+        st_s[(2 * j + 1) * kPWaves * 64] = l[j];
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+          o_s[(j * DT + d) * kPWaves * 64] = make_float4(o[j][d][0], o[j][d][1], o[j][d][2], o[j][d][3]);
+      }
+    }
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+      const float m0 = thr[j] == -INFINITY ? -INFINITY : -negref[j];
+      const float m1 = st_s[(2 * j) * kPWaves * 64];
+      const float top = fmaxf(m0, m1);
+      const float f0 = m0 == -INFINITY ? 0.f : fast_exp2(m0 - top);
+      const float f1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - top);
+      l[j] = l[j] * f0 + st_s[(2 * j + 1) * kPWaves * 64] * f1;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        const float4 x = o_s[(j * DT + d) * kPWaves * 64];
+        o[j][d] = o[j][d] * f0 + f4{x.x, x.y, x.z, x.w} * f1;
+      }
+    }
+  }
+
   // Row sums over the four lane groups, then O = O^T / l for the valid rows.
 #pragma unroll
   for (int j = 0; j < RT; ++j) {
@@ -648,23 +704,50 @@ __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(
   }
 }
 
+// Few tiles leave CUs idle or with one workgroup, and the launch then lasts as long as the
+// longest tile's chain of steps (0.68 us a step at Dh 128 with one wave per SIMD, against
+// 0.49 us with two).
+//  * At most one 128-row tile per CU, from kHalfTileKeys keys: 64-row tiles, each with two
+//    groups of waves (bf16, 32 / 8 heads, Dh 128: 256 tokens behind 4,000 cached ones 88 ->
+//    54 us, 16 chunks of up to 40 behind up to 4,096 78 -> 53 us, a 1,000-token prompt 27.5
+//    -> 24.2 us; 128-row tiles with two groups: 70, 68 and 25.5 us).
+//  * At most two, from kGroupKeys keys: 128-row tiles with two groups (the five ragged
+//    chunks of up to 777 behind up to 4,096, over e4m3 pools: 86 -> 70 us; 64-row tiles
+//    with one group 71 us). Below, the merge costs more than the shorter chain gives
+//    (four prompts of 400 to 500 tokens: 23.6 us, 27.6 with two groups).
+//  * More: 128-row tiles, one group.
+constexpr int64_t kCus = 256;
+constexpr int32_t kHalfTileKeys = 256;
+constexpr int32_t kGroupKeys = 1024;
+
+template <typename T, int DH, int G, int RT, int NG>
+int32_t launch_tiles(PrefillArgs a, int32_t num_seqs, int32_t num_kv_heads, int32_t max_query_len,
+                     hipStream_t s) {
+  a.num_kv_heads = num_kv_heads;
+  a.num_pairs = num_seqs * num_kv_heads;
+  a.tiles = static_cast<int32_t>(ceil_div(max_query_len, kPWaves * RT * 16 / G));
+  if (a.tiles == 0 || a.num_pairs == 0) return TKS_OK;
+  const int64_t groups = ceil_div(a.num_pairs, kXcds);
+  const dim3 grid(static_cast<unsigned>(groups * kXcds * a.tiles), 1, 1);
+  prefill_mfma_kernel<T, DH, G, RT, NG><<<grid, 64 * kPWaves * NG, 0, s>>>(a);
+  return check_launch();
+}
+
 template <typename T>
-int32_t launch_typed(const PrefillArgs &a, int32_t num_seqs, int32_t num_kv_heads, int32_t G,
-                     int32_t head_dim, int32_t max_query_len, hipStream_t s) {
-  constexpr int RT = 2;
-  constexpr int ROWS = kPWaves * RT * 16;
-#define TKS_PREFILL(DH, GG)                                                                  \
-  if (head_dim == DH && G == GG) {                                                           \
-    PrefillArgs args = a;                                                                    \
-    args.num_kv_heads = num_kv_heads;                                                        \
-    args.num_pairs = num_seqs * num_kv_heads;                                                \
-    args.tiles = static_cast<int32_t>(ceil_div(max_query_len, ROWS / GG));                   \
-    if (args.tiles == 0 || args.num_pairs == 0) return TKS_OK;                               \
-    const int64_t groups = ceil_div(args.num_pairs, kXcds);                                  \
-    const dim3 grid(static_cast<unsigned>(groups * kXcds * args.tiles), 1, 1);               \
-    prefill_mfma_kernel<T, DH, GG, RT><<<grid, 64 * kPWaves, 0, s>>>(args);                  \
-    return check_launch();                                                                   \
-  }
+int32_t launch_typed(const PrefillArgs &a, int32_t num_seqs, int64_t num_tokens,
+                     int32_t num_kv_heads, int32_t G, int32_t head_dim, int32_t max_query_len,
+                     hipStream_t s) {
+  // 128-row tiles of the batch, at most.
+  const int64_t tiles =
+      std::min(num_tokens * G / 128 + num_seqs,
+               num_seqs * ceil_div(static_cast<int64_t>(max_query_len) * G, 128)) * num_kv_heads;
+  const bool half = tiles <= kCus && a.key_cap >= kHalfTileKeys;
+  const bool two = tiles <= 2 * kCus && a.key_cap >= kGroupKeys;
+#define TKS_PREFILL(DH, GG)                                                                      \
+  if (head_dim == DH && G == GG)                                                                 \
+    return half  ? launch_tiles<T, DH, GG, 1, 2>(a, num_seqs, num_kv_heads, max_query_len, s)     \
+           : two ? launch_tiles<T, DH, GG, 2, 2>(a, num_seqs, num_kv_heads, max_query_len, s)     \
+                 : launch_tiles<T, DH, GG, 2, 1>(a, num_seqs, num_kv_heads, max_query_len, s);
   TKS_PREFILL(128, 4)
   TKS_PREFILL(128, 8)
   TKS_PREFILL(128, 1)
@@ -692,11 +775,11 @@ bool prefill_mfma_supported(int32_t dtype, int32_t head_dim, int32_t group, int3
 }
 
 int32_t launch_prefill_mfma(const PrefillArgs &a, int32_t dtype, int32_t num_seqs,
-                            int32_t num_kv_heads, int32_t group, int32_t head_dim,
+                            int64_t num_tokens, int32_t num_kv_heads, int32_t group, int32_t head_dim,
                             int32_t max_query_len, hipStream_t stream) {
   return dtype == TKS_BFLOAT16
-             ? launch_typed<bf16_t>(a, num_seqs, num_kv_heads, group, head_dim, max_query_len, stream)
-             : launch_typed<_Float16>(a, num_seqs, num_kv_heads, group, head_dim, max_query_len,
+             ? launch_typed<bf16_t>(a, num_seqs, num_tokens, num_kv_heads, group, head_dim, max_query_len, stream)
+             : launch_typed<_Float16>(a, num_seqs, num_tokens, num_kv_heads, group, head_dim, max_query_len,
                                       stream);
 }
 
