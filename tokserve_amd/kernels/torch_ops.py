@@ -3,8 +3,9 @@
 Each operator is declared with a schema that marks every tensor it writes
 (`Tensor(a!)`: KV pools, outputs, in-place rotations), has a CUDA-key kernel
 (HIP tensors dispatch as CUDA on ROCm) that hands the tensors' addresses,
-strides and the current stream to one `libtokserve_hip.so` entry point through
-the ctypes binding, and a fake (meta) kernel for tracing, so `torch.compile`,
+strides and the current stream to one `libtokserve_hip.so` entry point (natively,
+csrc/torch_ops.cpp, for the operators of an iteration, through the ctypes binding
+for the others), and a fake (meta) kernel for tracing, so `torch.compile`,
 FakeTensor propagation and HIP-graph capture all see the same operators. Every
 operator writes into tensors the caller passes (the validated wrappers in
 `ops.py` allocate them), so the fake kernels return nothing and the schemas need
@@ -34,6 +35,8 @@ kernels are Triton functions behind tokserve/kernels/<op>.py):
 """
 
 from __future__ import annotations
+
+from pathlib import Path
 
 import torch
 
@@ -240,31 +243,6 @@ def _decode_common(query, key_cache, value_cache, block_tables, seq_lens, seq_or
             pages_per_split, out.data_ptr(), out.stride(0), out.stride(1))
 
 
-def _paged_attention_decode(query, key_cache, value_cache, block_tables, seq_lens, seq_order,
-                            layer_index, max_seq_len, scale, pages_per_split, k_scale, v_scale,
-                            out, workspace_tensor, k_scales=None, v_scales=None):
-    _, _, num_kv_heads, block_size, head_dim = _pool_dims(key_cache)
-    if workspace_tensor is None:
-        nbytes = decode_workspace_bytes(query.shape[0], query.shape[1], num_kv_heads, head_dim,
-                                        block_size, max_seq_len, pages_per_split)
-        workspace_tensor = workspace(query.device, nbytes, "decode")
-    common = _decode_common(query, key_cache, value_cache, block_tables, seq_lens, seq_order,
-                            layer_index, max_seq_len, scale, pages_per_split, out)
-    ws = (_lib.ptr(workspace_tensor), 0 if workspace_tensor is None else workspace_tensor.numel())
-    library = _lib.load()
-    if k_scales is not None:
-        # The row entry takes the scale arrays right after the pools.
-        status = library.tks_paged_attention_decode_fp8_rows(
-            *common[:5], k_scales.data_ptr(), v_scales.data_ptr(), *common[5:], *ws,
-            _code(query), _stream(query))
-    elif key_cache.dtype == FP8_POOL_DTYPE:
-        status = library.tks_paged_attention_decode_fp8(*common, *ws, k_scale, v_scale,
-                                                        _code(query), _stream(query))
-    else:
-        status = library.tks_paged_attention_decode(*common, *ws, _code(query), _stream(query))
-    _lib.check(status, "paged_attention_decode")
-
-
 def _paged_attention_decode_noalloc(query, key_cache, value_cache, block_tables, seq_lens,
                                     seq_order, layer_index, max_seq_len, scale, pages_per_split,
                                     out):
@@ -273,50 +251,6 @@ def _paged_attention_decode_noalloc(query, key_cache, value_cache, block_tables,
     status = _lib.load().tks_paged_attention_decode_noalloc(*common, _code(query),
                                                             _stream(query))
     _lib.check(status, "paged_attention_decode_noalloc")
-
-
-def _paged_attention_prefill(query, key_cache, value_cache, block_tables, seq_lens,
-                             cu_seqlens_q, seq_order, layer_index, max_query_len, max_seq_len,
-                             scale, k_scale, v_scale, out, k_scales=None, v_scales=None):
-    dims = _pool_dims(key_cache)
-    num_seqs = seq_lens.shape[0]
-    common = (query.data_ptr(), query.stride(0), query.stride(1),
-              key_cache.data_ptr(), value_cache.data_ptr(), *dims, layer_index,
-              block_tables.data_ptr(), block_tables.shape[1], seq_lens.data_ptr(),
-              cu_seqlens_q.data_ptr(), _lib.ptr(seq_order), num_seqs, query.shape[0],
-              query.shape[1],
-              max_query_len, max_seq_len, scale, out.data_ptr(), out.stride(0), out.stride(1))
-    library = _lib.load()
-    if key_cache.dtype == FP8_POOL_DTYPE:
-        _, _, num_kv_heads, block_size, head_dim = dims
-        nbytes = library.tks_paged_attention_prefill_fp8_workspace_bytes(
-            num_seqs, query.shape[1], num_kv_heads, head_dim, block_size, block_tables.shape[1],
-            max_seq_len, _code(query))
-        if nbytes < 0:
-            raise ValueError("invalid fp8 prefill workspace query")
-        scratch = workspace(query.device, nbytes, "prefill_fp8_pages")
-        ws = (_lib.ptr(scratch), 0 if scratch is None else scratch.numel())
-        if k_scales is not None:
-            # The row entry takes the scale arrays right after the pools.
-            status = library.tks_paged_attention_prefill_fp8_rows(
-                *common[:5], k_scales.data_ptr(), v_scales.data_ptr(), *common[5:], *ws,
-                _code(query), _stream(query))
-        else:
-            status = library.tks_paged_attention_prefill_fp8(
-                *common, *ws, k_scale, v_scale, _code(query), _stream(query))
-    else:
-        status = library.tks_paged_attention_prefill(*common, _code(query), _stream(query))
-    _lib.check(status, "paged_attention_prefill")
-
-
-def _rms_norm(inputs, weight, epsilon, residual, out, residual_out):
-    status = _lib.load().tks_rms_norm(
-        inputs.data_ptr(), inputs.stride(0),
-        _lib.ptr(residual), 0 if residual is None else residual.stride(0),
-        _lib.ptr(residual_out), 0 if residual_out is None else residual_out.stride(0),
-        weight.data_ptr(), out.data_ptr(), out.stride(0), inputs.shape[0], inputs.shape[1],
-        epsilon, _code(inputs), _code(weight), _code(out), _stream(inputs))
-    _lib.check(status, "rms_norm")
 
 
 def _rope_launch(query, key, positions, cos, sin, query_out, key_out):
@@ -340,118 +274,30 @@ def _rope_inplace(query, key, positions, cos, sin):
     _rope_launch(query, key, positions, cos, sin, query, key)
 
 
-def _rope_kv_append_launch(query, query_out, key, value, positions, cos, sin, key_cache,
-                           value_cache, slot_mapping, layer_index, key_out, k_scale, v_scale,
-                           k_scales, v_scales):
-    num_layers, num_blocks, num_kv_heads, block_size, head_dim = _pool_dims(key_cache)
-    library = _lib.load()
-    fp8 = key_cache.dtype == FP8_POOL_DTYPE
-    pools = (key_cache.data_ptr(), value_cache.data_ptr())
-    if k_scales is not None:
-        entry, scales = library.tks_rope_kv_append_fp8_rows, ()
-        pools += (k_scales.data_ptr(), v_scales.data_ptr())
-    elif fp8:
-        entry, scales = library.tks_rope_kv_append_fp8, (k_scale, v_scale)
-    else:
-        entry, scales = library.tks_rope_kv_append, ()
-    status = entry(
-        query.data_ptr(), query_out.data_ptr(), query.stride(0), query.stride(1),
-        query_out.stride(0), query_out.stride(1), query.shape[1],
-        key.data_ptr(), _lib.ptr(key_out), key.stride(0), key.stride(1),
-        0 if key_out is None else key_out.stride(0), 0 if key_out is None else key_out.stride(1),
-        value.data_ptr(), value.stride(0), value.stride(1), num_kv_heads, query.shape[0],
-        head_dim, positions.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.shape[0],
-        *pools, num_layers, num_blocks, block_size,
-        layer_index, slot_mapping.data_ptr(), *scales, _code(query), _stream(query))
-    _lib.check(status, "rope_kv_append")
-
-
-def _rope_kv_append(query, key, value, positions, cos, sin, key_cache, value_cache,
-                    slot_mapping, layer_index, query_out, key_out, k_scale=1.0, v_scale=1.0,
-                    k_scales=None, v_scales=None):
-    _rope_kv_append_launch(query, query_out, key, value, positions, cos, sin, key_cache,
-                           value_cache, slot_mapping, layer_index, key_out, k_scale, v_scale,
-                           k_scales, v_scales)
-
-
-def _rope_kv_append_inplace(query, key, value, positions, cos, sin, key_cache, value_cache,
-                            slot_mapping, layer_index, key_out, k_scale=1.0, v_scale=1.0,
-                            k_scales=None, v_scales=None):
-    _rope_kv_append_launch(query, query, key, value, positions, cos, sin, key_cache,
-                           value_cache, slot_mapping, layer_index, key_out, k_scale, v_scale,
-                           k_scales, v_scales)
-
-
-def _rope_append_paged_decode(query, key, value, positions, cos, sin, slot_mapping, key_cache,
-                              value_cache, block_tables, seq_lens, seq_order, layer_index,
-                              max_seq_len, scale, pages_per_split, out, workspace_tensor,
-                              k_scale=1.0, v_scale=1.0, k_scales=None, v_scales=None):
-    num_layers, num_blocks, num_kv_heads, block_size, head_dim = _pool_dims(key_cache)
-    if workspace_tensor is None:
-        nbytes = decode_workspace_bytes(query.shape[0], query.shape[1], num_kv_heads, head_dim,
-                                        block_size, max_seq_len, pages_per_split)
-        workspace_tensor = workspace(query.device, nbytes, "decode")
-    library = _lib.load()
-    fp8 = key_cache.dtype == FP8_POOL_DTYPE
-    pools = (key_cache.data_ptr(), value_cache.data_ptr())
-    if k_scales is not None:
-        entry, scales = library.tks_rope_append_paged_decode_fp8_rows, ()
-        pools += (k_scales.data_ptr(), v_scales.data_ptr())
-    elif fp8:
-        entry, scales = library.tks_rope_append_paged_decode_fp8, (k_scale, v_scale)
-    else:
-        entry, scales = library.tks_rope_append_paged_decode, ()
-    status = entry(
-        query.data_ptr(), query.stride(0), query.stride(1),
-        key.data_ptr(), key.stride(0), key.stride(1),
-        value.data_ptr(), value.stride(0), value.stride(1),
-        positions.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.shape[0],
-        slot_mapping.data_ptr(), *pools,
-        num_layers, num_blocks, num_kv_heads, block_size, head_dim, layer_index,
-        block_tables.data_ptr(), block_tables.shape[1], seq_lens.data_ptr(), _lib.ptr(seq_order),
-        query.shape[0], query.shape[1], max_seq_len, scale, pages_per_split,
-        out.data_ptr(), out.stride(0), out.stride(1),
-        _lib.ptr(workspace_tensor), 0 if workspace_tensor is None else workspace_tensor.numel(),
-        *scales, _code(query), _stream(query))
-    _lib.check(status, "rope_append_paged_decode")
-
-
-def _greedy_argmax(logits, out):
-    status = _lib.load().tks_argmax(logits.data_ptr(), logits.stride(0), logits.shape[0],
-                                    logits.shape[1], out.data_ptr(), _code(logits),
-                                    _stream(logits))
-    _lib.check(status, "greedy_argmax")
-
-
-def _silu_mul(gate_up, out):
-    status = _lib.load().tks_silu_mul(gate_up.data_ptr(), gate_up.stride(0), gate_up.shape[0],
-                                      gate_up.shape[1] // 2, out.data_ptr(), out.stride(0),
-                                      _code(gate_up), _stream(gate_up))
-    _lib.check(status, "silu_mul")
-
-
 def _vector_add(x, y, out):
     status = _lib.load().tks_vector_add(x.data_ptr(), y.data_ptr(), out.data_ptr(), x.numel(),
                                         _code(x), _stream(x))
     _lib.check(status, "vector_add")
 
 
+# Operators with a device kernel here; the others' are native (csrc/torch_ops.cpp).
 KERNELS = {
     "kv_append": _kv_append,
     "paged_gather": _paged_gather,
-    "paged_attention_decode": _paged_attention_decode,
     "paged_attention_decode_noalloc": _paged_attention_decode_noalloc,
-    "paged_attention_prefill": _paged_attention_prefill,
-    "rms_norm": _rms_norm,
     "rope": _rope,
     "rope_": _rope_inplace,
-    "rope_kv_append": _rope_kv_append,
-    "rope_kv_append_": _rope_kv_append_inplace,
-    "rope_append_paged_decode": _rope_append_paged_decode,
-    "greedy_argmax": _greedy_argmax,
-    "silu_mul": _silu_mul,
     "vector_add": _vector_add,
 }
+
+NATIVE_LIBRARY = Path(__file__).resolve().parent.parent / "libtokserve_torch.so"
+
+
+def _not_built(*args, **kwargs) -> None:
+    raise RuntimeError(
+        f"{NATIVE_LIBRARY.name} is not built at {NATIVE_LIBRARY}; run "
+        "`python -c 'import __graft_entry__ as g; g.build()'` or `make -C tokserve_amd/csrc`"
+    )
 
 
 def _fake(*args, **kwargs) -> None:
@@ -464,8 +310,11 @@ def _register() -> None:
     library = torch.library.Library(NAMESPACE, "DEF")
     for name, schema in SCHEMAS.items():
         library.define(schema)
-        library.impl(name, KERNELS[name], "CUDA")
+        if name in KERNELS or not NATIVE_LIBRARY.is_file():
+            library.impl(name, KERNELS.get(name, _not_built), "CUDA")
         torch.library.register_fake(f"{NAMESPACE}::{name}", _fake, lib=library)
+    if NATIVE_LIBRARY.is_file():
+        torch.ops.load_library(str(NATIVE_LIBRARY))
     # Kept for the life of the process: dropping the handle would deregister the ops.
     globals()["_LIBRARY"] = library
 
