@@ -125,3 +125,18 @@ def test_fused_step_over_long_blocks_equals_its_two_calls(device, pool) -> None:
         if pool == "rows":
             for name in kw:
                 assert torch.equal(kw[name].nan_to_num(-1.0), kw2[name].nan_to_num(-1.0))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_infinite_values_past_a_waves_first_page_ids(device, dtype) -> None:
+    """An infinite value among more pages than a wave holds ids of at once (64): the wave
+    takes all of its pages again. Rounding as above; 1e-4 absolute for sums of 9,000 keys."""
+
+    batch = workloads.paged_batch([9000, 40], [1, 1], num_q_heads=8, num_kv_heads=2, head_dim=64,
+                                  block_size=32, dtype=dtype, device=device, seed=4)
+    for key in (5, 8990):
+        block = int(batch.block_tables[0, key // 32])
+        batch.value_cache[0, block, :, key % 32, key % 64] = float("inf")
+    out = _decode(batch, pages_per_split=1000).cpu()
+    assert_close(out.float(), _oracle(batch), rtol=ROUNDING[dtype], atol=1e-4)
+    assert torch.isinf(out[0, :, [5, 8990 % 64]]).all()

@@ -17,6 +17,8 @@
 #include "attention_common.hpp"
 #include "rope_common.hpp"
 
+#include <type_traits>
+
 namespace tks {
 namespace {
 
@@ -608,17 +610,23 @@ constexpr int kPvMinWaves = DH == 64 ? 3 : 1;
 // LONG: blocks of a.block_pages > 1 pages. Every page lies at a multiple of its own size
 // behind the KV head's first row, so a wave's page ids are kept in place of its block
 // ids and nothing else of the page loop changes. These shapes came from the VALU kernel
-// (paged_attention.hip), which keeps the probabilities in fp32, so here P.V keeps them
-// too: v_mfma_f32_16x16x4_f32, whose k-th operand lane group g holds element g for
-// instruction e, i.e. token 4 g + e, the very layout of the scores and of V^T as read.
-// Four such MFMAs per 16 dims instead of one of 16-bit operands: 1,024 cycles per page
-// and wave at Dh 128, hidden behind the four waves' page loads. 48 fp16 sequences of up
-// to 4,096 keys over blocks of 32 (32 / 8 heads, Dh 128, 359 MB): 81 us, 4.4 TB/s
-// (1,605 us with the VALU kernel), with its error against 64 bits.
+// (paged_attention.hip), which keeps the probabilities in fp32, so here P.V keeps their
+// 24 bits: as the sum of three bf16 values, or of two fp16 ones (22 bits; the reference is
+// moved down by kShift = 7 so that values down to 2^-31 keep bits), each part one 16-bit
+// MFMA. fp16 queries over pools with row
+// scales, which multiply the probabilities and may leave fp16's range, use
+// v_mfma_f32_16x16x4_f32 instead, whose k-th operand lane group g holds element g for
+// instruction e, i.e. token 4 g + e: the very layout of the scores and of V^T as read, but
+// four times the cycles of two parts. 48 fp16 sequences of up to 4,096 keys over blocks of 32 (32 / 8
+// heads, Dh 128, 359 MB): 1,605 us with the VALU kernel, 81 us with fp32 MFMAs, 71 us so,
+// the error against 64 bits the same.
 template <typename T, typename KV, int DH, int G, bool ROPE, bool ROWS, bool LONG>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kPvMinWaves<DH>)))
 void decode_pv_kernel(DecodeArgs a) {
   constexpr bool kFp8 = sizeof(KV) == 1;
+  constexpr bool kHalf = std::is_same<T, _Float16>::value;
+  constexpr int kParts = !LONG || (kHalf && ROWS) ? 0 : kHalf ? 2 : 3;
+  constexpr float kShift = kParts == 2 ? 7.f : 0.f;
   static_assert(!ROWS || kFp8, "row scales: fp8 pools");
   constexpr int BS = 16, NC = DH / 32, DT = DH / 16, CPR = DH / 8;
   constexpr int kPage = BS * DH;                        // elements of one K (or V) page
@@ -827,6 +835,7 @@ void decode_pv_kernel(DecodeArgs a) {
   // 0 while m is -inf), l = this lane's share of the sum (its tokens of each page).
   float m = -INFINITY, l = 0.f, thr = -INFINITY, mref = 0.f;
   const float scale_log2 = a.scale_log2;
+  bool whole = false;  // kParts: P.V with whole probabilities (a second pass, see below)
 
   // Page idx of the chunk's page-id register into ring slot SLOT: its K tile, then
   // its V tile (2 L loads, in that order).
@@ -967,7 +976,7 @@ void decode_pv_kernel(DecodeArgs a) {
       const float alpha = bump ? fast_exp2(m - mx) : 1.f;
       m = bump ? mx : m;
       thr = m + 8.f;
-      mref = m == -INFINITY ? 0.f : m;
+      mref = m == -INFINITY ? 0.f : m - kShift;
       l *= alpha;
 #pragma unroll
       for (int t = 0; t < DT; ++t)
@@ -982,10 +991,15 @@ void decode_pv_kernel(DecodeArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) pv[i] *= vs4[i];
     }
-    v4 pb;
-    if constexpr (!LONG) {
+    v4 pb[kParts > 0 ? kParts : 1];  // the probabilities, or their parts
 #pragma unroll
-      for (int i = 0; i < 4; ++i) pb[i] = static_cast<typename M::elem>(pv[i]);
+    for (int i = 0; i < 4; ++i) {
+      float rest = pv[i];
+#pragma unroll
+      for (int k = 0; k < (kParts > 0 ? kParts : 1); ++k) {
+        pb[k][i] = static_cast<typename M::elem>(rest);
+        rest -= static_cast<float>(pb[k][i]);
+      }
     }
     Reads::wait(vt);
     if (tail) {
@@ -1022,55 +1036,74 @@ void decode_pv_kernel(DecodeArgs a) {
     for (int t = 0; t < DT; ++t) {
       v4 vop;
       __builtin_memcpy(&vop, &vt[t], 8);
-      if constexpr (LONG) {
+      if (kParts > 0 && !whole) {
+#pragma unroll
+        for (int k = 0; k < kParts; ++k) acc[t] = M::run16(vop, pb[k], acc[t]);
+      } else if constexpr (LONG) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           acc[t] = mfma_f32(static_cast<float>(vop[e]), pv[e], acc[t]);
       } else {
-        acc[t] = M::run16(vop, pb, acc[t]);
+        acc[t] = M::run16(vop, pb[0], acc[t]);
       }
     }
   };
 
-  for (int c0 = w_begin; c0 < w_end; c0 += 64) {
-    const int n = min(w_end, c0 + 64) - c0;
-    int page_reg = 0;  // lane i: the id of page c0 + i, its block clamped into the pool
-    if (lane < n) {
-      const int at = LONG ? (c0 + lane) / block_pages : c0 + lane;
-      const int in_block = LONG ? c0 + lane - at * block_pages : 0;
-      page_reg = (int)block_of(bt_row, at, a.pool.num_blocks) * page_stride + in_block;
-    }
-    // The block ids, and everything else, before any page load is in flight: the
-    // waits below count only page loads.
-    __builtin_amdgcn_s_waitcnt(0);
-    issue(IntConst<0>{}, page_reg, 0);
-    if (D > 2 && n > 1) issue(IntConst<1 % D>{}, page_reg, 1);
-    int i = 0;  // page i sits in ring slot i % D
-    // Steady state: D pages per iteration, each consumed with the next D - 1 in flight.
-    for (; i + 2 * D - 1 <= n; i += D) {
-      issue(IntConst<(D - 1) % D>{}, page_reg, i + D - 1);
-      consume(BoolConst<false>{}, IntConst<0>{}, c0 + i, D - 1);
-      issue(IntConst<D % D>{}, page_reg, i + D);
-      consume(BoolConst<false>{}, IntConst<1 % D>{}, c0 + i + 1, D - 1);
+  for (;;) {
+    for (int c0 = w_begin; c0 < w_end; c0 += 64) {
+      const int n = min(w_end, c0 + 64) - c0;
+      int page_reg = 0;  // lane i: the id of page c0 + i, its block clamped into the pool
+      if (lane < n) {
+        const int at = LONG ? (c0 + lane) / block_pages : c0 + lane;
+        const int in_block = LONG ? c0 + lane - at * block_pages : 0;
+        page_reg = (int)block_of(bt_row, at, a.pool.num_blocks) * page_stride + in_block;
+      }
+      // The block ids, and everything else, before any page load is in flight: the
+      // waits below count only page loads.
+      __builtin_amdgcn_s_waitcnt(0);
+      issue(IntConst<0>{}, page_reg, 0);
+      if (D > 2 && n > 1) issue(IntConst<1 % D>{}, page_reg, 1);
+      int i = 0;  // page i sits in ring slot i % D
+      // Steady state: D pages per iteration, each consumed with the next D - 1 in flight.
+      for (; i + 2 * D - 1 <= n; i += D) {
+        issue(IntConst<(D - 1) % D>{}, page_reg, i + D - 1);
+        consume(BoolConst<false>{}, IntConst<0>{}, c0 + i, D - 1);
+        issue(IntConst<D % D>{}, page_reg, i + D);
+        consume(BoolConst<false>{}, IntConst<1 % D>{}, c0 + i + 1, D - 1);
+        if constexpr (D > 2) {
+          issue(IntConst<(D + 1) % D>{}, page_reg, i + D + 1);
+          consume(BoolConst<false>{}, IntConst<2 % D>{}, c0 + i + 2, D - 1);
+        }
+      }
+      // Fewer than 2 D - 1 pages left; those before i + D - 1 are in flight.
+      auto drain = [&](auto j_c) {
+        constexpr int j = decltype(j_c)::value;
+        if (i + j < n) {
+          if (i + j + D - 1 < n) issue(IntConst<(j + D - 1) % D>{}, page_reg, i + j + D - 1);
+          consume(BoolConst<true>{}, IntConst<j % D>{}, c0 + i + j, min(D - 1, n - 1 - (i + j)));
+        }
+      };
+      drain(IntConst<0>{});
+      drain(IntConst<1>{});
       if constexpr (D > 2) {
-        issue(IntConst<(D + 1) % D>{}, page_reg, i + D + 1);
-        consume(BoolConst<false>{}, IntConst<2 % D>{}, c0 + i + 2, D - 1);
+        drain(IntConst<2>{});
+        drain(IntConst<3>{});
       }
     }
-    // Fewer than 2 D - 1 pages left; those before i + D - 1 are in flight.
-    auto drain = [&](auto j_c) {
-      constexpr int j = decltype(j_c)::value;
-      if (i + j < n) {
-        if (i + j + D - 1 < n) issue(IntConst<(j + D - 1) % D>{}, page_reg, i + j + D - 1);
-        consume(BoolConst<true>{}, IntConst<j % D>{}, c0 + i + j, min(D - 1, n - 1 - (i + j)));
-      }
-    };
-    drain(IntConst<0>{});
-    drain(IntConst<1>{});
-    if constexpr (D > 2) {
-      drain(IntConst<2>{});
-      drain(IntConst<3>{});
-    }
+    if (kParts == 0 || whole) break;
+    // A value that is not finite times a probability's parts is NaN where the probability
+    // itself gives an infinity (parts may be 0 or negative): once more with whole ones.
+    bool nan = false;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) nan = nan || acc[t][i] != acc[t][i];
+    if (__builtin_amdgcn_ballot_w64(nan) == 0) break;
+    whole = true;
+    m = thr = -INFINITY;
+    l = mref = 0.f;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
   }
 
   // The staged rows to the pool, once this wave has read the page that holds their slot.
