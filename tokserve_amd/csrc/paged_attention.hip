@@ -409,6 +409,11 @@ __global__ __launch_bounds__(128) void merge_splits_kernel(
 //    more: 512-key splits (32 / 64 such Llama-3-8B sequences with the
 //    MFMA P.V kernel, split and merge: 45.3 / 90.5 us at 512 keys, 47.6 / 91.2 at
 //    1,024, 74.1 / 110.7 unsplit).
+//    e4m3 pools, half the bytes per key, under 16-bit queries: 1,280 keys (decode_impl;
+//    33 / 64 / 100 / 120 such sequences over pools with row scales: 38.1 / 63.7 / 94.5 /
+//    112.7 us at 512 keys, 33.4 / 56.7 / 84.5 / 98.0 at 1,280, 36.0 / 59.2 / 88.1 / 103.7
+//    at 768, 32.6 / 56.6 / 86.8 / 100.4 at 1,536; lengths uniform up to 8,192, per-pool
+//    scales: 33 / 64 / 100 take 54.9 / 104.2 / 166.9 at 512, 51.7 / 95.9 / 149.5 at 1,280).
 //  * Otherwise unsplit: 128, 192 and 256 Llama-3-8B sequences (128: 161.4 us
 //    against 166.2 at 1,024 keys and 173.3 at 512; 192: 216.4 against 249.6+ split),
 //    and short contexts (128 sequences x 4 KV heads, Dh 64, contexts up to 1152
@@ -419,6 +424,7 @@ constexpr int64_t kMaxFillSplitUnits = 48;
 constexpr int64_t kSplitBelowItems = 1024;
 constexpr int64_t kSplitUnits = 32;
 constexpr int64_t kSplitFromUnits = 256;
+constexpr int64_t kSplitKeysFp8 = 1280;
 constexpr int32_t kWideKeys = 640;  // fp32: see decode_impl
 
 int32_t split_unit(int32_t block_size) { return block_size % 16 == 0 ? 16 : block_size; }
@@ -583,14 +589,23 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
   if (!query || !key_cache || !value_cache || !block_tables || !seq_lens || !out)
     return TKS_ERR_VALUE;
 
-  const int32_t pps =
-      choose_pages_per_split(num_seqs, num_kv_heads, block_size, max_seq_len, pages_per_split,
-                             split_unit(block_size));
-  const int32_t max_splits = split_count(max_seq_len, block_size, pps);
+  int32_t pps = choose_pages_per_split(num_seqs, num_kv_heads, block_size, max_seq_len,
+                                       pages_per_split, split_unit(block_size));
+  int32_t max_splits = split_count(max_seq_len, block_size, pps);
   if (max_splits > kMaxGridSplits) return TKS_ERR_VALUE;
   Workspace w = carve(workspace, num_seqs, num_q_heads, max_splits, head_dim);
   if (max_splits > 1 && (workspace == nullptr || workspace_bytes < w.bytes))
     return TKS_ERR_WORKSPACE;
+  const bool mfma = mfma_eligible(dtype, num_blocks, num_kv_heads, block_size, head_dim, G, query,
+                                  q_seq_stride, q_head_stride, key_cache, value_cache, out,
+                                  out_seq_stride, out_head_stride);
+  if (mfma && fp8_pools && pages_per_split == 0 && max_splits > 1 &&
+      static_cast<int64_t>(num_seqs) * num_kv_heads >= kFillItems &&
+      static_cast<int64_t>(pps) * block_size < kSplitKeysFp8) {
+    pps = static_cast<int32_t>(ceil_div(kSplitKeysFp8, block_size));
+    max_splits = split_count(max_seq_len, block_size, pps);
+    w = carve(workspace, num_seqs, num_q_heads, max_splits, head_dim);
+  }
   const int32_t key_cap = static_cast<int32_t>(
       std::min<int64_t>(block_table_stride, static_cast<int64_t>(max_splits) * pps) * block_size);
 
@@ -598,9 +613,6 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float scale_log2 = scale * kLog2e * k_scale;
 
-  const bool mfma = mfma_eligible(dtype, num_blocks, num_kv_heads, block_size, head_dim, G, query,
-                                  q_seq_stride, q_head_stride, key_cache, value_cache, out,
-                                  out_seq_stride, out_head_stride);
   const bool f32 = dtype == TKS_FLOAT32 &&
                    decode_f32_supported(head_dim, G, block_size, num_blocks, num_kv_heads) &&
                    aligned16(query) && aligned16(key_cache) && aligned16(value_cache) &&
