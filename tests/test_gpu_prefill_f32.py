@@ -101,3 +101,21 @@ def test_prefill_f32_values_past_a_row_do_not_reach_it(device, dh, bad) -> None:
     hit[30:60, :, dh - 3] = True
     assert not bool(got[hit].isfinite().any())
     assert_close(got[~hit], clean[~hit], **TOL)
+
+
+@pytest.mark.parametrize("pool", ["same", "fp8_rows"])
+@pytest.mark.parametrize(("contexts", "chunks"),
+                         [([496, 90], [20, 28]), ([512, 90], [20, 28]), ([600, 90], [20, 29])])
+def test_prefill_f32_few_rows_over_many_keys(device, contexts, chunks, pool) -> None:
+    """Both sides of the rule that leaves few rows over many keys to the VALU kernel: below 512
+    keys and from there on, 48 and 49 tokens of 32 heads x 128."""
+
+    kw = dict(kv_dtype=torch.float8_e4m3fn, scale_granularity="row") if pool != "same" else {}
+    batch = workloads.paged_batch(contexts, chunks, num_q_heads=32, num_kv_heads=8, head_dim=128,
+                                  block_size=16, dtype=torch.float32, device=device, seed=6, **kw)
+    got = _run(batch, batch.key_cache, batch.value_cache, **batch.scale_kwargs)
+    pools = []
+    for cache, scales in ((batch.key_cache, batch.k_scales), (batch.value_cache, batch.v_scales)):
+        rows = cache.cpu().double()
+        pools.append(rows if scales is None else rows * scales.cpu().double().unsqueeze(-1))
+    assert_close(got, _oracle(batch, *pools), **TOL)

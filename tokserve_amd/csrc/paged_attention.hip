@@ -425,6 +425,8 @@ constexpr int64_t kSplitBelowItems = 1024;
 constexpr int64_t kSplitUnits = 32;
 constexpr int64_t kSplitFromUnits = 256;
 constexpr int64_t kSplitKeysFp8 = 1280;
+constexpr int64_t kFewElements = int64_t{3} << 16;  // fp32 prefill: see prefill_impl
+constexpr int32_t kFewKeys = 512;
 constexpr int32_t kWideKeys = 640;  // fp32: see decode_impl
 
 int32_t split_unit(int32_t block_size) { return block_size % 16 == 0 ? 16 : block_size; }
@@ -812,9 +814,19 @@ int32_t prefill_impl(const void *query, int64_t q_token_stride, int64_t q_head_s
   }
   const int kv_elem = fp8_pools ? 1 : elem_bytes(dtype);
   // fp32 queries: fp32 products on the matrix cores (16 prompts of 64 to 1,024 tokens,
-  // 32 / 4 heads, Dh 64: 828 us on the VALU kernel below, 124 us). Row maxima of raw
-  // scores again need a positive scale.
-  if (dtype == TKS_FLOAT32 && scale_log2 > 0.f && scale_log2 < INFINITY &&
+  // 32 / 4 heads, Dh 64: 825 us on the VALU kernel below, 117 us). Row maxima of raw
+  // scores again need a positive scale. Few rows over many keys stay on the VALU kernel,
+  // whose four waves share a row's keys where a tile's chain of steps is one wave's: up to
+  // kFewElements query elements and two VALU workgroups per CU, from kFewKeys keys. Of 32
+  // / 8 heads, Dh 128, 32 tokens in four chunks: 40 us (VALU) and 34 us at 300 keys, 82
+  // and 102 at 1,000, 281 and 386 at 4,000; 64 tokens in one: 508 and 378 us at 4,000. Of
+  // 8 / 2, Dh 64, 200 tokens: 139 and 226 us at 4,000; 512 in eight: 273 and 220 us. (Over
+  // e4m3 pools at Dh 128 the VALU kernel reads V a byte at a time: 555 and 384 us for the
+  // four chunks, so only up to 16 of its workgroups go there: one token, 347 and 361 us.)
+  const bool few = num_tokens * num_kv_heads <= 2 * kFillItems &&
+                   num_tokens * num_q_heads * head_dim <= kFewElements && key_cap >= kFewKeys &&
+                   (!fp8_pools || head_dim <= 64 || num_tokens * num_kv_heads <= 16);
+  if (dtype == TKS_FLOAT32 && !few && scale_log2 > 0.f && scale_log2 < INFINITY &&
       prefill_f32_supported(head_dim, G) && aligned16(query) && aligned16(out) &&
       aligned16(key_cache) && aligned16(value_cache) && q_token_stride % 4 == 0 &&
       q_head_stride % 4 == 0 && out_token_stride % 4 == 0 && out_head_stride % 4 == 0) {
