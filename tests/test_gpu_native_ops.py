@@ -1,5 +1,5 @@
-"""The operators' native device kernels: errors as _lib.check raises them, and split partials
-that belong to one call."""
+"""The operators' native device kernels: errors as _lib.check raises them, and scratch memory
+that belongs to one call."""
 
 import pytest
 import torch
@@ -49,6 +49,41 @@ def test_split_decodes_on_two_streams_keep_their_partials_apart(device) -> None:
         for i, batch in enumerate(batches):
             with torch.cuda.stream(streams[i]):
                 outs[i].append(decode(batch))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(out, expected[i]) for out in outs[i])
+
+
+@pytest.mark.parametrize("granularity", ["pool", "row"])
+def test_fp8_prefills_on_two_streams_keep_their_pages_apart(device, granularity) -> None:
+    """The decoded pages of a call are its own: nothing per device is kept for them, and calls
+    on two streams give what they give alone."""
+
+    kw = (dict(scale_granularity="row") if granularity == "row"
+          else dict(k_scale=0.5, v_scale=0.25))
+    batches = [workloads.paged_batch([2000 + 300 * i, 90, 1300], [40, 90, 300], num_q_heads=32,
+                                     num_kv_heads=8, head_dim=128, block_size=16,
+                                     dtype=torch.bfloat16, device=device, seed=i,
+                                     kv_dtype=torch.float8_e4m3fn, **kw)
+               for i in range(2)]
+
+    def prefill(batch):
+        return ops.paged_attention_prefill(batch.query, batch.key_cache, batch.value_cache,
+                                           batch.block_tables, batch.seq_lens,
+                                           batch.cu_seqlens_q, layer_index=0,
+                                           max_query_len=batch.max_query_len,
+                                           max_seq_len=batch.max_seq_len, **batch.scale_kwargs)
+
+    kept = dict(torch_ops._workspaces)
+    expected = [prefill(batch) for batch in batches]
+    assert torch_ops._workspaces == kept
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in batches]
+    outs: list = [[], []]
+    for _ in range(10):
+        for i, batch in enumerate(batches):
+            with torch.cuda.stream(streams[i]):
+                outs[i].append(prefill(batch))
     torch.cuda.synchronize()
     for i in range(2):
         assert all(torch.equal(out, expected[i]) for out in outs[i])

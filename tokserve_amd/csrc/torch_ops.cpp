@@ -137,17 +137,21 @@ T *as(const OptTensor &t) { return static_cast<T *>(mut(t)); }
 int32_t i32(int64_t x) { return static_cast<int32_t>(x); }
 bool fp8(const Tensor &pool) { return pool.scalar_type() == at::kFloat8_e4m3fn; }
 
-// Split partials of a decode whose caller gave no workspace: from the caching allocator, on
-// the launch's stream (a buffer of its own for every call, also across streams and threads).
+// Scratch memory of one call, undefined for 0 bytes: from the caching allocator on the
+// launch's stream, so no other call, stream or thread shares it.
+Tensor scratch(int64_t bytes, const Tensor &query, const char *use) {
+  TORCH_CHECK_VALUE(bytes >= 0, "invalid ", use, " workspace query");
+  return bytes == 0 ? Tensor() : at::empty({bytes}, query.options().dtype(at::kByte));
+}
+
+// Split partials of a decode: the caller's workspace, or scratch.
 Tensor decode_workspace(const OptTensor &given, const Tensor &query, const Tensor &pool,
                         int64_t max_seq_len, int64_t pages_per_split) {
   if (given) return *given;
-  const int64_t bytes = library().tks_paged_attention_decode_workspace_bytes(
-      i32(query.size(0)), i32(query.size(1)), i32(pool.size(2)), i32(pool.size(4)),
-      i32(pool.size(3)), i32(max_seq_len), i32(pages_per_split));
-  TORCH_CHECK_VALUE(bytes >= 0, "invalid decode workspace query");
-  if (bytes == 0) return Tensor();
-  return at::empty({bytes}, query.options().dtype(at::kByte));
+  return scratch(library().tks_paged_attention_decode_workspace_bytes(
+                     i32(query.size(0)), i32(query.size(1)), i32(pool.size(2)), i32(pool.size(4)),
+                     i32(pool.size(3)), i32(max_seq_len), i32(pages_per_split)),
+                 query, "decode");
 }
 
 void paged_attention_decode(const Tensor &query, const Tensor &key_cache,
@@ -186,19 +190,13 @@ void paged_attention_decode(const Tensor &query, const Tensor &key_cache,
         "paged_attention_decode");
 }
 
-// torch_ops.workspace(): the per-device buffer the decoded pages of fp8 pools go to.
+// The decoded pages of fp8 pools.
 Tensor fp8_pages(const Tensor &query, const Tensor &pool, int64_t num_seqs, int64_t table_width,
                  int64_t max_seq_len) {
-  const int64_t bytes = library().tks_paged_attention_prefill_fp8_workspace_bytes(
-      i32(num_seqs), i32(query.size(1)), i32(pool.size(2)), i32(pool.size(4)), i32(pool.size(3)),
-      i32(table_width), i32(max_seq_len), code(query));
-  TORCH_CHECK_VALUE(bytes >= 0, "invalid fp8 prefill workspace query");
-  if (bytes == 0) return Tensor();
-  return with_python([&] {
-    return pybind11::module_::import("tokserve_amd.kernels.torch_ops")
-        .attr("workspace")(query.device(), bytes, "prefill_fp8_pages")
-        .cast<Tensor>();
-  });
+  return scratch(library().tks_paged_attention_prefill_fp8_workspace_bytes(
+                     i32(num_seqs), i32(query.size(1)), i32(pool.size(2)), i32(pool.size(4)),
+                     i32(pool.size(3)), i32(table_width), i32(max_seq_len), code(query)),
+                 query, "fp8 prefill");
 }
 
 void paged_attention_prefill(const Tensor &query, const Tensor &key_cache,

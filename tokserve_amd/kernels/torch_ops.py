@@ -157,10 +157,10 @@ def _pool_dims(pool: torch.Tensor) -> tuple[int, int, int, int, int]:
     return num_layers, num_blocks, num_kv_heads, block_size, head_dim
 
 
-# Per-(device, use) scratch buffers of the kernels that need one. They only grow;
-# a replaced buffer stays allocated, since a captured HIP graph keeps the device
-# address it was recorded with. Calls that share a buffer are ordered on one
-# stream, as the kernels require.
+# Per-(device, use) scratch buffers for callers that pass an operator a workspace of their
+# own (an operator given none allocates one for the call). They only grow; a replaced
+# buffer stays allocated, since a captured HIP graph keeps the device address it was
+# recorded with. Calls that share a buffer must be ordered on one stream.
 _workspaces: dict[tuple[torch.device, str], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
 
