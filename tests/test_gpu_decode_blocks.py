@@ -1,5 +1,5 @@
 """Decode over blocks of several 16-token pages (the MFMA decode keeps page ids there, and
-its probabilities in fp32) against the fp32 oracle, and the fused step against its two
+its probabilities at 24 bits) against the fp32 oracle, and the fused step against its two
 calls, bit for bit.
 
 Tolerance against the oracle: the result's one rounding to the stored dtype (half a step,
@@ -140,3 +140,31 @@ def test_infinite_values_past_a_waves_first_page_ids(device, dtype) -> None:
     out = _decode(batch, pages_per_split=1000).cpu()
     assert_close(out.float(), _oracle(batch), rtol=ROUNDING[dtype], atol=1e-4)
     assert torch.isinf(out[0, :, [5, 8990 % 64]]).all()
+
+
+@pytest.mark.parametrize("pool", ["pool", "fp8"])
+@pytest.mark.parametrize(("dtype", "dh"), [(torch.float16, 64), (torch.float16, 128),
+                                           (torch.bfloat16, 128)])
+def test_small_probabilities_keep_their_bits(device, dtype, dh, pool) -> None:
+    """One key of each page holds nearly all of the weight and a value of 0; the other keys, of
+    about e^-18 (2^-26) each, make up the whole result. An fp32 exponent of up to 27 is within
+    2^-19 relative, so the result's one rounding is all that shows."""
+
+    kw = dict(kv_dtype=FP8, k_scale=1.0, v_scale=16.0) if pool == "fp8" else {}
+    batch = workloads.paged_batch([8192, 1000], [1, 1], num_q_heads=8, num_kv_heads=2,
+                                  head_dim=dh, block_size=32, dtype=dtype, device=device, seed=6,
+                                  **kw)
+    top = (torch.arange(32, device=device) % 16 == 0)[:, None]
+    size = 1.125 if dh == 64 else 0.8125  # scores of -9 and 9, or about
+    batch.query.fill_(1.0)
+    batch.key_cache.copy_(torch.where(top, size, -size).expand(batch.key_cache.shape))
+    gen = torch.Generator().manual_seed(1)
+    values = 200 + 240 * torch.rand(batch.value_cache.shape, generator=gen).to(device)
+    batch.value_cache.copy_(torch.where(top, 0.0, values if pool == "fp8" else 16 * values))
+    pools = [cache.cpu().double() * scale for cache, scale in
+             ((batch.key_cache, batch.k_scale), (batch.value_cache, batch.v_scale))]
+    expected = paged.decode_batch(batch.query.cpu().double(), *pools, batch.block_tables.cpu(),
+                                  batch.seq_lens.cpu(), 0, torch.float64)
+    for pages_per_split in (0, 1000):
+        out = _decode(batch, pages_per_split=pages_per_split).cpu()
+        assert_close(out.double(), expected, rtol=ROUNDING[dtype], atol=0)

@@ -599,9 +599,10 @@ struct IntConst {
 // VGPRs (left to itself the compiler put them in AGPRs, with a copy per access:
 // fp8 serving shape 10.4 -> 10.0 us). At Dh 128 the budget is left alone: three
 // waves per SIMD over fp8 pools (145 VGPRs) ran the Llama-3-8B decode batch 3 %
-// slower (152.5 vs 148.7 us).
-template <int DH>
-constexpr int kPvMinWaves = DH == 64 ? 3 : 1;
+// slower (152.5 vs 148.7 us). Over long blocks two waves are asked for, which keeps the two
+// sets of sums of fp16's parts in VGPRs (48 fp16 sequences, in a graph: 85.1 -> 80.4 us).
+template <int DH, bool LONG>
+constexpr int kPvMinWaves = DH == 64 ? 3 : LONG ? 2 : 1;
 
 // ROWS: fp8 pools with one scale per pool row (a.k_rs, a.v_rs): a page's 16 K and 16
 // V scales ride in the ring with it; a lane multiplies its scores by its tokens' K
@@ -611,22 +612,26 @@ constexpr int kPvMinWaves = DH == 64 ? 3 : 1;
 // behind the KV head's first row, so a wave's page ids are kept in place of its block
 // ids and nothing else of the page loop changes. These shapes came from the VALU kernel
 // (paged_attention.hip), which keeps the probabilities in fp32, so here P.V keeps their
-// 24 bits: as the sum of three bf16 values, or of two fp16 ones (22 bits; the reference is
-// moved down by kShift = 7 so that values down to 2^-31 keep bits), each part one 16-bit
-// MFMA. fp16 queries over pools with row
-// scales, which multiply the probabilities and may leave fp16's range, use
-// v_mfma_f32_16x16x4_f32 instead, whose k-th operand lane group g holds element g for
-// instruction e, i.e. token 4 g + e: the very layout of the scores and of V^T as read, but
-// four times the cycles of two parts. 48 fp16 sequences of up to 4,096 keys over blocks of 32 (32 / 8
-// heads, Dh 128, 359 MB): 1,605 us with the VALU kernel, 81 us with fp32 MFMAs, 71 us so,
-// the error against 64 bits the same.
+// 24 bits, as three 16-bit parts with one MFMA each. bf16 parts have fp32's range and share
+// the accumulators. fp16 parts are scaled, p = h0 + 2^-11 h1 + 2^-22 h2, and the reference is
+// moved down by kShift = 7: exact for p from 2^-30 of the reference, within 2^-54 of it
+// below. The sums of h1 and h2 are kept apart from h0's (a page's of h2 is scaled into
+// h1's). fp16 queries over pools with row scales, which multiply the probabilities and may
+// leave fp16's range, use v_mfma_f32_16x16x4_f32 instead, whose k-th operand lane group g
+// holds element g for instruction e, i.e. token 4 g + e: the very layout of the scores and of
+// V^T as read, but 8 / 3 of the cycles of three parts. 48 fp16 sequences of up to 4,096 keys
+// over blocks of 32 (32 / 8 heads, Dh 128, 359 MB), in a graph: 80.4 us, 87.3 with fp32 MFMAs
+// (two parts, which lose bits, 76.4); the VALU kernel took 1,605 us. Over e4m3 pools 62.1,
+// 79.9 and 53.6 us.
 template <typename T, typename KV, int DH, int G, bool ROPE, bool ROWS, bool LONG>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kPvMinWaves<DH>)))
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kPvMinWaves<DH, LONG>)))
 void decode_pv_kernel(DecodeArgs a) {
   constexpr bool kFp8 = sizeof(KV) == 1;
   constexpr bool kHalf = std::is_same<T, _Float16>::value;
-  constexpr int kParts = !LONG || (kHalf && ROWS) ? 0 : kHalf ? 2 : 3;
-  constexpr float kShift = kParts == 2 ? 7.f : 0.f;
+  constexpr int kParts = !LONG || (kHalf && ROWS) ? 0 : 3;
+  constexpr bool kScaled = kHalf && kParts > 0;  // parts by their scale, each with its sums
+  constexpr float kShift = kScaled ? 7.f : 0.f;
+  constexpr float kPartScale = kScaled ? 2048.f : 1.f;
   static_assert(!ROWS || kFp8, "row scales: fp8 pools");
   constexpr int BS = 16, NC = DH / 32, DT = DH / 16, CPR = DH / 8;
   constexpr int kPage = BS * DH;                        // elements of one K (or V) page
@@ -829,6 +834,9 @@ void decode_pv_kernel(DecodeArgs a) {
   f4 acc[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+  f4 low[DT];  // kScaled: the sums of the second and third parts, by 2^11
+#pragma unroll
+  for (int t = 0; t < DT; ++t) low[t] = f4{0.f, 0.f, 0.f, 0.f};
   // Softmax state of head column r (equal in the column's four lanes): m = the
   // reference max in log2 units (-inf before the first key), thr = m + 8 (a score
   // above it moves the reference), mref = the value subtracted before exp2 (m, or
@@ -982,6 +990,10 @@ void decode_pv_kernel(DecodeArgs a) {
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[t][i] *= alpha;
+      if constexpr (kScaled) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t) low[t] *= alpha;
+      }
     }
     float pv[4];
 #pragma unroll
@@ -998,7 +1010,7 @@ void decode_pv_kernel(DecodeArgs a) {
 #pragma unroll
       for (int k = 0; k < (kParts > 0 ? kParts : 1); ++k) {
         pb[k][i] = static_cast<typename M::elem>(rest);
-        rest -= static_cast<float>(pb[k][i]);
+        rest = (rest - static_cast<float>(pb[k][i])) * kPartScale;
       }
     }
     Reads::wait(vt);
@@ -1037,8 +1049,14 @@ void decode_pv_kernel(DecodeArgs a) {
       v4 vop;
       __builtin_memcpy(&vop, &vt[t], 8);
       if (kParts > 0 && !whole) {
+        acc[t] = M::run16(vop, pb[0], acc[t]);
+        if constexpr (kScaled) {
+          low[t] = M::run16(vop, pb[1], low[t]);
+          low[t] += M::run16(vop, pb[2], f4{0.f, 0.f, 0.f, 0.f}) * (1.f / kPartScale);
+        } else {
 #pragma unroll
-        for (int k = 0; k < kParts; ++k) acc[t] = M::run16(vop, pb[k], acc[t]);
+          for (int k = 1; k < kParts; ++k) acc[t] = M::run16(vop, pb[k], acc[t]);
+        }
       } else if constexpr (LONG) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -1091,6 +1109,11 @@ void decode_pv_kernel(DecodeArgs a) {
       }
     }
     if (kParts == 0 || whole) break;
+    if constexpr (kScaled) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+        acc[t] += low[t] * (1.f / kPartScale);
+    }
     // A value that is not finite times a probability's parts is NaN where the probability
     // itself gives an infinity (parts may be 0 or negative): once more with whole ones.
     bool nan = false;
