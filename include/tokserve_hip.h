@@ -53,6 +53,7 @@ enum tks_status {
 };
 
 /* ABI version of this header; bumped on any signature change. */
+#define TKS_ABI_VERSION 12
 int32_t tks_abi_version(void);
 
 /* Static description of a status code (never NULL). */

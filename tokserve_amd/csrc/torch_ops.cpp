@@ -7,13 +7,16 @@
 // 5,060 and 4,270 us.
 //
 // The entry points are looked up in libtokserve_hip.so on the first call, so loading this
-// library does not touch HIP. Errors are raised by tokserve_amd.kernels._lib, which maps a
+// library does not touch HIP. It is loaded and registered by torch_ops.py, which first
+// compares the versions it was built against (of torch, and of the C ABI that it calls
+// through) with those it is loaded into. Errors are raised by tokserve_amd.kernels._lib, which maps a
 // status to its exception.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/library.h>
+#include <torch/headeronly/version.h>
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
@@ -351,13 +354,30 @@ void silu_mul(const Tensor &gate_up, const Tensor &out) {
 
 }  // namespace
 
-TORCH_LIBRARY_IMPL(tokserve_amd, CUDA, m) {
-  m.impl("paged_attention_decode", paged_attention_decode);
-  m.impl("paged_attention_prefill", paged_attention_prefill);
-  m.impl("rope_append_paged_decode", rope_append_paged_decode);
-  m.impl("rope_kv_append", rope_kv_append);
-  m.impl("rope_kv_append_", rope_kv_append_);
-  m.impl("rms_norm", rms_norm);
-  m.impl("greedy_argmax", greedy_argmax);
-  m.impl("silu_mul", silu_mul);
+extern "C" const char *tks_torch_built_for(void) { return TORCH_VERSION; }
+
+extern "C" int32_t tks_torch_abi_version(void) { return TKS_ABI_VERSION; }
+
+// Registers the device kernels, once; null, or why not.
+extern "C" const char *tks_torch_register(void) {
+  static std::string error;
+  try {
+    static const torch::Library kernels = [] {
+      torch::Library m(torch::Library::IMPL, "tokserve_amd", c10::DispatchKey::CUDA, __FILE__,
+                       __LINE__);
+      m.impl("paged_attention_decode", paged_attention_decode);
+      m.impl("paged_attention_prefill", paged_attention_prefill);
+      m.impl("rope_append_paged_decode", rope_append_paged_decode);
+      m.impl("rope_kv_append", rope_kv_append);
+      m.impl("rope_kv_append_", rope_kv_append_);
+      m.impl("rms_norm", rms_norm);
+      m.impl("greedy_argmax", greedy_argmax);
+      m.impl("silu_mul", silu_mul);
+      return m;
+    }();
+  } catch (const std::exception &raised) {
+    error = raised.what();
+    return error.c_str();
+  }
+  return nullptr;
 }

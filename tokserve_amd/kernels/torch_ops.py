@@ -36,6 +36,7 @@ kernels are Triton functions behind tokserve/kernels/<op>.py):
 
 from __future__ import annotations
 
+import ctypes
 from pathlib import Path
 
 import torch
@@ -293,11 +294,39 @@ KERNELS = {
 NATIVE_LIBRARY = Path(__file__).resolve().parent.parent / "libtokserve_torch.so"
 
 
-def _not_built(*args, **kwargs) -> None:
-    raise RuntimeError(
-        f"{NATIVE_LIBRARY.name} is not built at {NATIVE_LIBRARY}; run "
-        "`python -c 'import __graft_entry__ as g; g.build()'` or `make -C tokserve_amd/csrc`"
-    )
+def _load_native(path: Path) -> str | None:
+    """Registers the native device kernels; None, or why it could not (the package then imports
+    all the same, also under another torch or a CPU-only one)."""
+
+    rebuild = ("; run `python -c 'import __graft_entry__ as g; g.build()'` or "
+               "`make -C tokserve_amd/csrc`")
+    if not path.is_file():
+        return f"{path.name} is not built at {path}{rebuild}"
+    try:
+        library = ctypes.CDLL(str(path))
+        library.tks_torch_built_for.restype = ctypes.c_char_p
+        library.tks_torch_register.restype = ctypes.c_char_p
+        torch_version = library.tks_torch_built_for().decode()
+        abi_version = library.tks_torch_abi_version()
+    except (OSError, AttributeError) as error:
+        return f"{path} does not load into torch {torch.__version__} ({error}){rebuild}"
+    if torch_version != torch.__version__.split("+")[0]:
+        return (f"{path} was built for torch {torch_version}, not {torch.__version__}"
+                f"{rebuild}")
+    if abi_version != _lib.ABI_VERSION:
+        return (f"{path} ABI {abi_version} does not match binding {_lib.ABI_VERSION}"
+                f"{rebuild}")
+    error = library.tks_torch_register()
+    return None if error is None else f"{path}: {error.decode()}{rebuild}"
+
+
+def _unavailable(reason: str):
+    """A device kernel that raises."""
+
+    def kernel(*args, **kwargs) -> None:
+        raise RuntimeError(reason)
+
+    return kernel
 
 
 def _fake(*args, **kwargs) -> None:
@@ -310,11 +339,13 @@ def _register() -> None:
     library = torch.library.Library(NAMESPACE, "DEF")
     for name, schema in SCHEMAS.items():
         library.define(schema)
-        if name in KERNELS or not NATIVE_LIBRARY.is_file():
-            library.impl(name, KERNELS.get(name, _not_built), "CUDA")
         torch.library.register_fake(f"{NAMESPACE}::{name}", _fake, lib=library)
-    if NATIVE_LIBRARY.is_file():
-        torch.ops.load_library(str(NATIVE_LIBRARY))
+    missing = _load_native(NATIVE_LIBRARY)
+    for name in SCHEMAS:
+        if name in KERNELS:
+            library.impl(name, KERNELS[name], "CUDA")
+        elif missing is not None:
+            library.impl(name, _unavailable(missing), "CUDA")
     # Kept for the life of the process: dropping the handle would deregister the ops.
     globals()["_LIBRARY"] = library
 
