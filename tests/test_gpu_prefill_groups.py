@@ -56,3 +56,16 @@ def test_prefill_two_groups_per_tile(device, hq, hkv, dh, lengths) -> None:
     _check(device, torch.bfloat16, hq, hkv, dh, lengths)
     order = torch.tensor([3, 0, 4, 1, 2], dtype=torch.int32, device=device)
     _check(device, torch.float16, hq, hkv, dh, lengths, seq_order=order)
+
+
+# 32 / 8 heads at Dh 128, around one and two rounds of two-group workgroups: one sequence on each
+# side of the rules by its mean keys, ragged chunks over more than one round, and chunks that
+# stay with one group for their keys or their number.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lengths", [
+    ([569], [569]), ([1051], [569]), ([1972], [569]), ([1323], [1323]), ([2100], [1323]),
+    ([3267, 1419, 556, 1209, 1969], [233, 385, 198, 88, 254]),
+    ([1700, 1650, 1601, 1500, 1, 1690], [266, 257, 289, 290, 1, 260]),
+    ([2100, 2050, 400], [700, 700, 400])])
+def test_prefill_forms(device, dtype, lengths) -> None:
+    _check(device, dtype, 32, 8, 128, lengths)

@@ -228,7 +228,7 @@ constexpr int kPrefillOccupancy = DH == 64 ? 4 : 2;
 // NG = 2 splits a tile's steps between two groups of kPWaves waves (even and odd steps),
 // each with its own ring and sums, merged through LDS at the end: batches with fewer tiles
 // than CUs can hold last as long as their longest tile's chain of steps, which this halves
-// (launch_typed's rule).
+// (tile_form's rules).
 template <typename T, int DH, int G, int RT, int NG>
 __global__ __launch_bounds__(64 * kPWaves * NG) __attribute__((amdgpu_waves_per_eu(
     kPrefillOccupancy<DH>, kPrefillOccupancy<DH>))) void prefill_mfma_kernel(PrefillArgs a) {
@@ -706,19 +706,64 @@ __global__ __launch_bounds__(64 * kPWaves * NG) __attribute__((amdgpu_waves_per_
 
 // Few tiles leave CUs idle or with one workgroup, and the launch then lasts as long as the
 // longest tile's chain of steps (0.68 us a step at Dh 128 with one wave per SIMD, against
-// 0.49 us with two).
-//  * At most one 128-row tile per CU, from kHalfTileKeys keys: 64-row tiles, each with two
-//    groups of waves (bf16, 32 / 8 heads, Dh 128: 256 tokens behind 4,000 cached ones 88 ->
-//    54 us, 16 chunks of up to 40 behind up to 4,096 78 -> 53 us, a 1,000-token prompt 27.5
-//    -> 24.2 us; 128-row tiles with two groups: 70, 68 and 25.5 us).
-//  * At most two, from kGroupKeys keys: 128-row tiles with two groups (the five ragged
-//    chunks of up to 777 behind up to 4,096, over e4m3 pools: 86 -> 70 us; 64-row tiles
-//    with one group 71 us). Below, the merge costs more than the shorter chain gives
-//    (four prompts of 400 to 500 tokens: 23.6 us, 27.6 with two groups).
-//  * More: 128-row tiles, one group.
-constexpr int64_t kCus = 256;
+// 0.49 us with two). Two groups of waves halve the chain; 64-row tiles do less per step, but
+// need twice the workgroups. What decides is whether the workgroups of the busiest XCD (all
+// tiles of a pair run on one XCD, of 32 CUs) run at once: with two groups one per CU at Dh
+// 128, two at Dh 64. Of the time of 128-row tiles with one group, over 1,374 bf16 batches of
+// 1 to 16 chunks (32 / 8 heads at Dh 128; 32 / 4 and 8 / 2 at Dh 64), chunks and cached
+// lengths alike or ragged:
+//  * Half tiles with two groups, from kHalfTileKeys keys. Dh 128: while they run at once,
+//    0.62 - 0.98 (with up to two rounds of them 0.63 - 1.25); a single sequence's, which
+//    start with few keys under the causal mask, count by their mean keys. Dh 64: up to one
+//    128-row tile per CU in all and two rounds on an XCD, 0.48 - 1.03 (more rounds 0.71 - 1.20).
+//  * Whole tiles with two groups. While they run at once, from kGroupKeys keys, 0.68 - 1.0
+//    (a full round of them at Dh 128 from kTwoRoundKeys only: 0.84 - 1.11, 1.31 with fewer).
+//    In up to two rounds at Dh 64 from kTwoRoundKeys keys, 0.69 - 1.10 (where an XCD has one
+//    pair, up to 5 / 4 of a round: above, 0.87 - 1.09). In up to 3 / 2 rounds at Dh 128 from
+//    kRaggedKeys keys: 0.78 - 1.08 of batches whose cached lengths differ, 0.76 - 1.14 of
+//    batches where they are alike, which the host cannot tell; from kTwoRoundKeys 0.73 - 1.20.
+//    A single sequence again by its mean keys, 0.84 - 1.03.
+//  * Else whole tiles with one group.
 constexpr int32_t kHalfTileKeys = 256;
-constexpr int32_t kGroupKeys = 1024;
+constexpr int32_t kTwoRoundKeys = 1024;
+constexpr int32_t kRaggedKeys = 2048;
+template <int DH>
+constexpr int32_t kGroupKeys = DH == 128 ? 512 : 1024;
+
+struct TileForm {
+  bool half, groups;
+};
+
+template <int DH>
+TileForm tile_form(int64_t num_seqs, int64_t num_tokens, int64_t Hkv, int64_t G,
+                   int64_t max_query_len, int64_t keys) {
+  constexpr TileForm kHalf{true, true}, kGroups{false, true}, kWhole{false, false};
+  constexpr int64_t room = DH == 128 ? 32 : 64;  // workgroups of two groups per XCD
+  const int64_t pairs = num_seqs * Hkv;
+  // Tiles of `rows` rows, at most: on the busiest XCD, and in all.
+  auto busiest = [&](int64_t rows) {
+    return std::min(ceil_div(pairs, kXcds) * ceil_div(max_query_len * G, rows),
+                    ceil_div(Hkv, kXcds) * (num_tokens * G / rows + num_seqs));
+  };
+  const int64_t all = Hkv * std::min(num_tokens * G / 128 + num_seqs,
+                                     num_seqs * ceil_div(max_query_len * G, 128));
+  const int64_t halves = busiest(64), wholes = busiest(128);
+  if constexpr (DH == 64) {
+    if (keys >= kHalfTileKeys && all <= 8 * 32 && halves <= 2 * room) return kHalf;
+    if (keys >= kTwoRoundKeys && all <= 2 * 8 * 32 && (pairs > kXcds || 4 * wholes <= 5 * room))
+      return kGroups;
+    return kWhole;
+  }
+  // One sequence's tiles need from keys - max_query_len to keys keys.
+  const bool one = num_seqs == 1;
+  const int64_t mean = one ? std::max(keys / 2, keys - max_query_len / 2) : keys;
+  if (keys >= kHalfTileKeys && halves * mean <= room * keys) return kHalf;
+  if (keys >= kGroupKeys<DH> && wholes < room) return kGroups;
+  if (keys >= kTwoRoundKeys && (wholes <= room || (one && wholes * mean <= room * keys)))
+    return kGroups;
+  if (keys >= kRaggedKeys && !one && 2 * wholes <= 3 * room) return kGroups;
+  return kWhole;
+}
 
 template <typename T, int DH, int G, int RT, int NG>
 int32_t launch_tiles(PrefillArgs a, int32_t num_seqs, int32_t num_kv_heads, int32_t max_query_len,
@@ -733,21 +778,23 @@ int32_t launch_tiles(PrefillArgs a, int32_t num_seqs, int32_t num_kv_heads, int3
   return check_launch();
 }
 
+template <typename T, int DH, int G>
+int32_t launch_form(const PrefillArgs &a, int32_t num_seqs, int64_t num_tokens,
+                    int32_t num_kv_heads, int32_t max_query_len, hipStream_t s) {
+  const TileForm form =
+      tile_form<DH>(num_seqs, num_tokens, num_kv_heads, G, max_query_len, a.key_cap);
+  return form.half     ? launch_tiles<T, DH, G, 1, 2>(a, num_seqs, num_kv_heads, max_query_len, s)
+         : form.groups ? launch_tiles<T, DH, G, 2, 2>(a, num_seqs, num_kv_heads, max_query_len, s)
+                       : launch_tiles<T, DH, G, 2, 1>(a, num_seqs, num_kv_heads, max_query_len, s);
+}
+
 template <typename T>
 int32_t launch_typed(const PrefillArgs &a, int32_t num_seqs, int64_t num_tokens,
                      int32_t num_kv_heads, int32_t G, int32_t head_dim, int32_t max_query_len,
                      hipStream_t s) {
-  // 128-row tiles of the batch, at most.
-  const int64_t tiles =
-      std::min(num_tokens * G / 128 + num_seqs,
-               num_seqs * ceil_div(static_cast<int64_t>(max_query_len) * G, 128)) * num_kv_heads;
-  const bool half = tiles <= kCus && a.key_cap >= kHalfTileKeys;
-  const bool two = tiles <= 2 * kCus && a.key_cap >= kGroupKeys;
-#define TKS_PREFILL(DH, GG)                                                                      \
-  if (head_dim == DH && G == GG)                                                                 \
-    return half  ? launch_tiles<T, DH, GG, 1, 2>(a, num_seqs, num_kv_heads, max_query_len, s)     \
-           : two ? launch_tiles<T, DH, GG, 2, 2>(a, num_seqs, num_kv_heads, max_query_len, s)     \
-                 : launch_tiles<T, DH, GG, 2, 1>(a, num_seqs, num_kv_heads, max_query_len, s);
+#define TKS_PREFILL(DH, GG)      \
+  if (head_dim == DH && G == GG) \
+    return launch_form<T, DH, GG>(a, num_seqs, num_tokens, num_kv_heads, max_query_len, s);
   TKS_PREFILL(128, 4)
   TKS_PREFILL(128, 8)
   TKS_PREFILL(128, 1)
