@@ -118,3 +118,21 @@ def test_decode_f32_fused_step_equals_its_two_calls(device, hq, hkv, dh, block_s
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int32), expected.view(torch.int32))
     assert torch.equal(batch.key_cache, k_ref) and torch.equal(batch.value_cache, v_ref)
+
+
+@pytest.mark.parametrize("pool", ["same", "fp8_rows"])
+@pytest.mark.parametrize(("dh", "hkv", "seqs", "keys"), [
+    (64, 2, 8, 640), (64, 2, 8, 641), (128, 8, 3, 384), (128, 8, 3, 385), (128, 8, 16, 640),
+    (128, 8, 17, 640), (128, 8, 17, 641)])
+def test_decode_f32_unsplit_or_split(device, dh, hkv, seqs, keys, pool) -> None:
+    """Both sides of the lines up to which a small batch runs unsplit (8 waves to a pair)."""
+
+    contexts = [keys] + [1 + (37 * i) % keys for i in range(seqs - 1)]
+    batch = _batch(device, contexts, 4 * hkv, hkv, dh, 16, pool)
+    expected = _oracle(batch)
+    _poison(batch, pool)
+    out = ops.paged_attention_decode(batch.query, batch.key_cache, batch.value_cache,
+                                     batch.block_tables, batch.seq_lens, layer_index=0,
+                                     max_seq_len=keys, **batch.scale_kwargs)
+    torch.cuda.synchronize()
+    assert_close(out.cpu(), expected, **TOL)

@@ -405,8 +405,8 @@ __global__ __launch_bounds__(128) void merge_splits_kernel(
 //    keys (8 / 16 Llama-3-8B sequences x 8
 //    KV heads, contexts log-uniform in [128, 8192]: 39.3 / 41.8 us at 1,024 keys,
 //    34.8 / 37.0 us at 768, 39.3 / 45.9 us at 256; 16 sequences unsplit: 59 us).
-//  * Fewer than kSplitBelowItems pairs and a length bound of kSplitFromKeys or
-//    more: 512-key splits (32 / 64 such Llama-3-8B sequences with the
+//  * Fewer than kSplitBelowItems pairs and a length bound of kSplitFromUnits * 16
+//    or more: 512-key splits (32 / 64 such Llama-3-8B sequences with the
 //    MFMA P.V kernel, split and merge: 45.3 / 90.5 us at 512 keys, 47.6 / 91.2 at
 //    1,024, 74.1 / 110.7 unsplit).
 //    e4m3 pools, half the bytes per key, under 16-bit queries: 1,280 keys (decode_impl;
@@ -428,6 +428,7 @@ constexpr int64_t kSplitKeysFp8 = 1280;
 constexpr int64_t kFewElements = int64_t{3} << 16;  // fp32 prefill: see prefill_impl
 constexpr int32_t kFewKeys = 512;
 constexpr int32_t kWideKeys = 640;  // fp32: see decode_impl
+constexpr int32_t kWideKeys128 = 384;
 
 int32_t split_unit(int32_t block_size) { return block_size % 16 == 0 ? 16 : block_size; }
 
@@ -666,12 +667,20 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
   }
 
   int32_t st;
-  // A small fp32 batch of short sequences runs unsplit, with more waves per workgroup, and
-  // saves the merge launch. One CU then does a pair's products, so only while they are
-  // short: 8 sequences x 2 KV heads, Dh 64, cold: 14 us up to 513 keys and 19.5 us up to
-  // 1,024, against 9.6 us and a merge of 4.7 us.
-  const bool wide = f32 && pages_per_split == 0 && max_splits > 1 && max_seq_len <= kWideKeys &&
-                    static_cast<int64_t>(num_seqs) * num_kv_heads < kFillItems;
+  // A small fp32 batch of short sequences runs unsplit, with eight waves per workgroup, and
+  // saves the merge launch; one CU then does a pair's products, twice as many at Dh 128. Against
+  // splits and merge, each eager / in a graph, us:
+  //   Dh 64, 16 pairs    512 keys 11.7 / 11.2 and 14.1 / 11.4, 630 keys 13.7 / 13.2 and 14.0 / 11.5
+  //   Dh 64, 128 pairs   512 keys 13.3 / 12.9 and 14.2 / 12.9, 630 keys 15.3 / 15.2 and 14.9 / 14.1
+  //   Dh 128, 16 pairs   375 keys - / 16.3 and - / 18.2, 512 keys 21.8 / 21.5 and 19.4 / 18.8
+  //   Dh 128, 128 pairs  375 keys - / 20.2 and - / 21.1, 512 keys 24.0 / 25.9 and 22.3 / 22.0
+  // (e4m3 pools at Dh 128, 64 pairs, in a graph: 375 keys 12.7 and 14.0, 440 keys 15.2 and
+  // 14.2.) Past kFillItems / 2 pairs the splits are halves, and more than there are CUs: 630
+  // keys of 248 pairs take 33.3 us at Dh 128, split 38.8.
+  const int64_t pairs = static_cast<int64_t>(num_seqs) * num_kv_heads;
+  const bool wide = f32 && pages_per_split == 0 && max_splits > 1 && pairs < kFillItems &&
+                    max_seq_len <= (head_dim <= 64 || 2 * pairs > kFillItems ? kWideKeys
+                                                                             : kWideKeys128);
   const int32_t splits = wide ? 1 : max_splits;
   if (mfma || f32) {
     DecodeArgs a{query,      q_seq_stride, q_head_stride, key_cache,   value_cache,
