@@ -119,3 +119,29 @@ def test_prefill_f32_few_rows_over_many_keys(device, contexts, chunks, pool) -> 
         rows = cache.cpu().double()
         pools.append(rows if scales is None else rows * scales.cpu().double().unsqueeze(-1))
     assert_close(got, _oracle(batch, *pools), **TOL)
+
+
+def test_prefill_f32_more_workgroups_than_a_launch_holds(device) -> None:
+    """2,048 chunks of four tokens under a bound of 8,192, 16 KV heads: a tile for every
+    sequence, KV head and 16 tokens of the bound are 2^24 workgroups, 2^32 threads, one more
+    than a launch may have. The VALU kernel, a workgroup per token, takes them."""
+
+    seqs, hq, hkv, dh = 2048, 64, 16, 64
+    batch = workloads.paged_batch([4 + i % 29 for i in range(seqs)], [4] * seqs, num_q_heads=hq,
+                                  num_kv_heads=hkv, head_dim=dh, block_size=16,
+                                  dtype=torch.float32, device=device, seed=8,
+                                  pool_on_device_rng=True)
+    tables = torch.zeros((seqs, 512), dtype=torch.int32, device=device)
+    tables[:, :batch.block_tables.shape[1]] = batch.block_tables
+    out = ops.paged_attention_prefill(
+        batch.query, batch.key_cache, batch.value_cache, tables, batch.seq_lens,
+        batch.cu_seqlens_q, layer_index=0, max_query_len=8192, max_seq_len=8192)
+    # (the same chunks 64 at a time, which the other work order takes)
+    for first in range(0, seqs, 64 * 8):
+        part = slice(first, first + 64)
+        rows = slice(4 * first, 4 * (first + 64))
+        expected = ops.paged_attention_prefill(
+            batch.query[rows], batch.key_cache, batch.value_cache, batch.block_tables[part],
+            batch.seq_lens[part], batch.cu_seqlens_q[first:first + 65] - 4 * first, layer_index=0,
+            max_query_len=4, max_seq_len=32)
+        assert_close(out[rows], expected, **TOL)

@@ -363,7 +363,8 @@ int32_t launch_prefill_mfma(const PrefillArgs &a, int32_t dtype, int32_t num_seq
 
 // The fp32 prefill on the matrix cores (16-byte aligned rows, scale_log2 > 0), over fp32
 // or e4m3 pools; returns a tks_status.
-bool prefill_f32_supported(int32_t head_dim, int32_t group);
+bool prefill_f32_supported(int32_t head_dim, int32_t group, int64_t num_seqs, int64_t num_tokens,
+                           int64_t num_kv_heads, int64_t max_query_len);
 int32_t launch_prefill_f32(const PrefillArgs &a, int32_t num_seqs, int64_t num_tokens,
                            int32_t num_kv_heads, int32_t group, int32_t head_dim,
                            int32_t max_query_len, bool fp8_pools, hipStream_t stream);

@@ -836,7 +836,8 @@ int32_t prefill_impl(const void *query, int64_t q_token_stride, int64_t q_head_s
                    num_tokens * num_q_heads * head_dim <= kFewElements && key_cap >= kFewKeys &&
                    (!fp8_pools || head_dim <= 64 || num_tokens * num_kv_heads <= 16);
   if (dtype == TKS_FLOAT32 && !few && scale_log2 > 0.f && scale_log2 < INFINITY &&
-      prefill_f32_supported(head_dim, G) && aligned16(query) && aligned16(out) &&
+      prefill_f32_supported(head_dim, G, num_seqs, num_tokens, num_kv_heads, max_query_len) &&
+      aligned16(query) && aligned16(out) &&
       aligned16(key_cache) && aligned16(value_cache) && q_token_stride % 4 == 0 &&
       q_head_stride % 4 == 0 && out_token_stride % 4 == 0 && out_head_stride % 4 == 0) {
     PrefillArgs p{query,    q_token_stride, q_head_stride, key_cache,    value_cache,

@@ -22,6 +22,8 @@
 // probabilities). Rows are padded by 16 bytes against bank conflicts.
 #include "attention_common.hpp"
 
+#include <algorithm>
+
 namespace tks {
 namespace {
 
@@ -431,10 +433,25 @@ int32_t launch_f32(const PrefillArgs &a, int32_t G, int32_t head_dim, dim3 grid,
   return check_launch();
 }
 
+int64_t prefill_f32_blocks(int64_t num_seqs, int64_t num_tokens, int64_t num_kv_heads, int32_t group,
+                           int64_t max_query_len) {
+  const int64_t qt = kFRows / group;
+  // Tiles of n sequences with N tokens in all: at most N / QT + n. (A chunk longer than the
+  // batch's tokens does not exist: max_query_len may be a loose bound.)
+  return num_seqs <= kTileOrderSeqs
+             ? (num_tokens / qt + num_seqs) * num_kv_heads
+             : num_seqs * num_kv_heads * ceil_div(std::min(max_query_len, num_tokens), qt);
+}
+
 }  // namespace
 
-bool prefill_f32_supported(int32_t head_dim, int32_t group) {
-  return (head_dim == 64 || head_dim == 128) && group >= 1 && group <= 16;
+bool prefill_f32_supported(int32_t head_dim, int32_t group, int64_t num_seqs, int64_t num_tokens,
+                           int64_t num_kv_heads, int64_t max_query_len) {
+  return (head_dim == 64 || head_dim == 128) && group >= 1 && group <= 16 &&
+         num_seqs * num_kv_heads <= INT32_MAX &&
+         // A launch has fewer than 2^32 threads.
+         prefill_f32_blocks(num_seqs, num_tokens, num_kv_heads, group, max_query_len) <
+             (int64_t{1} << 32) / (64 * kFWaves);
 }
 
 int32_t launch_prefill_f32(const PrefillArgs &a, int32_t num_seqs, int64_t num_tokens,
@@ -444,13 +461,11 @@ int32_t launch_prefill_f32(const PrefillArgs &a, int32_t num_seqs, int64_t num_t
   args.num_kv_heads = num_kv_heads;
   args.num_seqs = num_seqs;
   args.num_pairs = num_seqs * num_kv_heads;
-  args.tiles = static_cast<int32_t>(ceil_div(max_query_len, kFRows / group));
+  args.tiles = static_cast<int32_t>(
+      ceil_div(std::min<int64_t>(max_query_len, num_tokens), kFRows / group));
   if (args.tiles == 0 || args.num_pairs == 0) return TKS_OK;
-  // Tiles of n sequences with N tokens in all: at most N / QT + n.
   const int64_t blocks =
-      num_seqs <= kTileOrderSeqs
-          ? (num_tokens / (kFRows / group) + num_seqs) * static_cast<int64_t>(num_kv_heads)
-          : static_cast<int64_t>(args.num_pairs) * args.tiles;
+      prefill_f32_blocks(num_seqs, num_tokens, num_kv_heads, group, max_query_len);
   const dim3 grid(static_cast<unsigned>(blocks));
   if (!fp8_pools) return launch_f32<float, false>(args, group, head_dim, grid, stream);
   return a.k_rs != nullptr ? launch_f32<fp8e4m3_t, true>(args, group, head_dim, grid, stream)
