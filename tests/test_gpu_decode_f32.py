@@ -136,3 +136,26 @@ def test_decode_f32_unsplit_or_split(device, dh, hkv, seqs, keys, pool) -> None:
                                      max_seq_len=keys, **batch.scale_kwargs)
     torch.cuda.synchronize()
     assert_close(out.cpu(), expected, **TOL)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize(("hq", "dh"), [(8, 64), (6, 128)])
+def test_decode_f32_values_that_are_not_finite(device, hq, dh, bad) -> None:
+    """A value that is not finite under a visible key reaches its dimension of that sequence and
+    KV head as it is, and no other result, wherever the key lies among waves and splits."""
+
+    contexts = [400, 400, 33]
+    batch = _batch(device, contexts, hq, 2, dh, 16, "same")
+    clean = _oracle(batch)
+    group = hq // 2
+    hit = torch.zeros(clean.shape, dtype=torch.bool)
+    for b, key, head, dim in ((0, 5, 0, 3), (0, 399, 0, dh - 1), (1, 200, 1, 17), (2, 32, 1, 0)):
+        block = int(batch.block_tables[b, key // 16])
+        batch.value_cache[0, block, head, key % 16, dim] = bad
+        hit[b, head * group:(head + 1) * group, dim] = True
+    for pages_per_split in (0, 1, 3, 1000):
+        out = ops.paged_attention_decode(batch.query, batch.key_cache, batch.value_cache,
+                                         batch.block_tables, batch.seq_lens, layer_index=0,
+                                         max_seq_len=400, pages_per_split=pages_per_split).cpu()
+        assert_close(out[hit], torch.full_like(out[hit], bad), rtol=0, atol=0, equal_nan=True)
+        assert_close(out[~hit], clean[~hit], **TOL)

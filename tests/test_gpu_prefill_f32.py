@@ -145,3 +145,56 @@ def test_prefill_f32_more_workgroups_than_a_launch_holds(device) -> None:
             batch.seq_lens[part], batch.cu_seqlens_q[first:first + 65] - 4 * first, layer_index=0,
             max_query_len=4, max_seq_len=32)
         assert_close(out[rows], expected, **TOL)
+
+
+@pytest.mark.parametrize("pool", ["same", "fp8_rows"])
+@pytest.mark.parametrize("seqs", [64, 65, 100])
+def test_prefill_f32_many_sequences(device, seqs, pool) -> None:
+    """Up to 64 sequences the tiles are found in the order of their keys, past that level by
+    level: empty chunks, chunks of one and of several tiles, with and without an order."""
+
+    chunks = [(0, 1, 17, 40, 5, 130, 16)[i % 7] for i in range(seqs)]
+    contexts = [q + (0, 3, 250, 31)[i % 4] for i, q in enumerate(chunks)]
+    kw = dict(kv_dtype=torch.float8_e4m3fn, scale_granularity="row") if pool != "same" else {}
+    batch = workloads.paged_batch(contexts, chunks, num_q_heads=8, num_kv_heads=2, head_dim=64,
+                                  block_size=16, dtype=torch.float32, device=device, seed=seqs,
+                                  **kw)
+    pools = []
+    for cache, scales in ((batch.key_cache, batch.k_scales), (batch.value_cache, batch.v_scales)):
+        rows = cache.cpu().double()
+        pools.append(rows if scales is None else rows * scales.cpu().double().unsqueeze(-1))
+    expected = _oracle(batch, *pools)
+    for order in (None, ops.longest_first(contexts, device)):
+        got = _run(batch, batch.key_cache, batch.value_cache, seq_order=order,
+                   **batch.scale_kwargs)
+        assert_close(got, expected, **TOL)
+
+
+@pytest.mark.parametrize("pool", ["fp8", "fp8_rows"])
+@pytest.mark.parametrize(("hq", "dh"), [(8, 64), (2, 128), (16, 128)])
+def test_prefill_f32_codes_past_a_row_do_not_reach_it(device, hq, dh, pool) -> None:
+    """The same over e4m3 pools: a NaN code reaches its dimension of the rows that see its key,
+    an infinite row scale every dimension of them, and no other row."""
+
+    kw = (dict(k_scale=0.5, v_scale=0.25) if pool == "fp8" else dict(scale_granularity="row"))
+    batch = workloads.paged_batch([100, 90], [60, 90], num_q_heads=hq, num_kv_heads=1, head_dim=dh,
+                                  block_size=16, dtype=torch.float32, device=device, seed=5,
+                                  kv_dtype=torch.float8_e4m3fn, **kw)
+    pools = []
+    for cache, scale, scales in ((batch.key_cache, batch.k_scale, batch.k_scales),
+                                 (batch.value_cache, batch.v_scale, batch.v_scales)):
+        rows = cache.cpu().double()
+        pools.append(rows * (scale if scales is None else scales.cpu().double().unsqueeze(-1)))
+    clean = _oracle(batch, *pools)
+    key = 70  # query token 30 of the first chunk
+    at = (0, int(batch.block_tables[0, key // 16]), 0, key % 16)
+    hit = torch.zeros(clean.shape, dtype=torch.bool)
+    if pool == "fp8":
+        batch.value_cache.view(torch.uint8)[(*at, dh - 3)] = 0x7F
+        hit[30:60, :, dh - 3] = True
+    else:
+        batch.v_scales[at] = float("inf")
+        hit[30:60] = True
+    got = _run(batch, batch.key_cache, batch.value_cache, **batch.scale_kwargs)
+    assert not bool(got[hit].isfinite().any())
+    assert_close(got[~hit], clean[~hit], **TOL)
