@@ -1,6 +1,6 @@
-"""16-bit decode over e4m3 pools with the library's own, longer key splits (256 to 1,023
-(sequence, KV head) pairs and a bound of 4,096 keys or more) against the fp32 oracle:
-lengths around the 1,280-key splits and blocks that do not divide them.
+"""16-bit decode over e4m3 pools with the library's own key splits (256 to 1,023 (sequence, KV
+head) pairs and a bound of 4,096 keys or more) against the fp32 oracle: lengths around the
+splits, of 1,280 keys or, for fewer pairs at Dh 64, 512, and blocks that do not divide them.
 
 The keys at the ends of splits, pages and sequences have values of 64 among N(0, 1) ones: one of
 them left out or taken twice moves a result by about 64 / 4,100 or more, several tolerances.
@@ -20,15 +20,16 @@ from tokserve_amd.kernels import ops
 pytestmark = pytest.mark.gpu
 
 CONTEXTS = [4100, 1279, 1280, 1281, 2560, 2561, 1, 0] + [17 + 61 * i for i in range(56)]
+SPLITS = {4: 512, 8: 1280}  # KV heads of the 64 sequences: keys per split
 LARGE = 64.0
 
 
-def _mark(batch, block_size: int) -> None:
+def _mark(batch, block_size: int, split: int) -> None:
     """Values of +-LARGE (by dim) at the first and last keys of splits and sequences."""
 
     tables = batch.block_tables.cpu()
     for b, n in enumerate(batch.contexts):
-        ends = {p for e in range(0, n, 1280) for p in (e - 16, e - 1, e, e + 15)} | {n - 1}
+        ends = {p for e in range(0, n, split) for p in (e - 16, e - 1, e, e + 15)} | {n - 1}
         for p in sorted(p for p in ends if 0 <= p < n):
             block, row = int(tables[b, p // block_size]), p % block_size
             sign = torch.where(torch.arange(batch.value_cache.shape[4]) % 3 == p % 3, -1.0, 1.0)
@@ -43,13 +44,15 @@ def _mark(batch, block_size: int) -> None:
 
 @pytest.mark.parametrize("granularity", ["pool", "row"])
 @pytest.mark.parametrize("block_size", [16, 48])
-def test_fp8_decode_splits(device, granularity, block_size) -> None:
+@pytest.mark.parametrize("kv_heads", [4, 8])
+def test_fp8_decode_splits(device, granularity, block_size, kv_heads) -> None:
     kw = (dict(scale_granularity="row") if granularity == "row"
           else dict(k_scale=0.5, v_scale=0.25))
-    batch = workloads.paged_batch(CONTEXTS, [1] * len(CONTEXTS), num_q_heads=8, num_kv_heads=4,
-                                  head_dim=64, block_size=block_size, dtype=torch.bfloat16,
-                                  device=device, seed=2, kv_dtype=torch.float8_e4m3fn, **kw)
-    _mark(batch, block_size)
+    batch = workloads.paged_batch(CONTEXTS, [1] * len(CONTEXTS), num_q_heads=2 * kv_heads,
+                                  num_kv_heads=kv_heads, head_dim=64, block_size=block_size,
+                                  dtype=torch.bfloat16, device=device, seed=2,
+                                  kv_dtype=torch.float8_e4m3fn, **kw)
+    _mark(batch, block_size, SPLITS[kv_heads])
     out = ops.paged_attention_decode(
         batch.query, batch.key_cache, batch.value_cache, batch.block_tables, batch.seq_lens,
         layer_index=0, max_seq_len=batch.max_seq_len, **batch.scale_kwargs)

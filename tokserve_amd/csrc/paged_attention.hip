@@ -409,11 +409,12 @@ __global__ __launch_bounds__(128) void merge_splits_kernel(
 //    or more: 512-key splits (32 / 64 such Llama-3-8B sequences with the
 //    MFMA P.V kernel, split and merge: 45.3 / 90.5 us at 512 keys, 47.6 / 91.2 at
 //    1,024, 74.1 / 110.7 unsplit).
-//    e4m3 pools, half the bytes per key, under 16-bit queries: 1,280 keys (decode_impl;
-//    33 / 64 / 100 / 120 such sequences over pools with row scales: 38.1 / 63.7 / 94.5 /
-//    112.7 us at 512 keys, 33.4 / 56.7 / 84.5 / 98.0 at 1,280, 36.0 / 59.2 / 88.1 / 103.7
-//    at 768, 32.6 / 56.6 / 86.8 / 100.4 at 1,536; lengths uniform up to 8,192, per-pool
-//    scales: 33 / 64 / 100 take 54.9 / 104.2 / 166.9 at 512, 51.7 / 95.9 / 149.5 at 1,280).
+//    e4m3 pools, half the bytes per key, under 16-bit queries: 1,280 keys (decode_impl), at Dh
+//    64 from kSplitItemsFp8 pairs. Of the time at 512 keys, 256 to 512 pairs, lengths alike,
+//    uniform and log-uniform up to 4,200 - 8,192, both kinds of scales: Dh 128 (32 / 8 heads)
+//    0.86 - 1.05, mean 0.96 (33 log-uniform sequences, row scales: 38.1 us at 512 keys, 36.0 at 768,
+//    37.5 at 1,024, 33.4 at 1,280, 32.6 at 1,536); Dh 64 (32 / 4 and 16 / 8) 0.90 - 1.04, mean 0.96 from
+//    448 pairs, 0.87 - 1.33, mean 1.02 below.
 //  * Otherwise unsplit: 128, 192 and 256 Llama-3-8B sequences (128: 161.4 us
 //    against 166.2 at 1,024 keys and 173.3 at 512; 192: 216.4 against 249.6+ split),
 //    and short contexts (128 sequences x 4 KV heads, Dh 64, contexts up to 1152
@@ -425,6 +426,7 @@ constexpr int64_t kSplitBelowItems = 1024;
 constexpr int64_t kSplitUnits = 32;
 constexpr int64_t kSplitFromUnits = 256;
 constexpr int64_t kSplitKeysFp8 = 1280;
+constexpr int64_t kSplitItemsFp8 = 448;
 constexpr int64_t kFewElements = int64_t{3} << 16;  // fp32 prefill: see prefill_impl
 constexpr int32_t kFewKeys = 512;
 constexpr int32_t kWideKeys = 640;  // fp32: see decode_impl
@@ -603,7 +605,8 @@ int32_t decode_impl(const void *query, int64_t q_seq_stride, int64_t q_head_stri
                                   q_seq_stride, q_head_stride, key_cache, value_cache, out,
                                   out_seq_stride, out_head_stride);
   if (mfma && fp8_pools && pages_per_split == 0 && max_splits > 1 &&
-      static_cast<int64_t>(num_seqs) * num_kv_heads >= kFillItems &&
+      static_cast<int64_t>(num_seqs) * num_kv_heads >=
+          (head_dim <= 64 ? kSplitItemsFp8 : kFillItems) &&
       static_cast<int64_t>(pps) * block_size < kSplitKeysFp8) {
     pps = static_cast<int32_t>(ceil_div(kSplitKeysFp8, block_size));
     max_splits = split_count(max_seq_len, block_size, pps);
