@@ -61,29 +61,30 @@ def test_prefill_f32_shapes(device, hq, hkv, dh, block_size, pool) -> None:
     assert_close(got, _oracle(batch, keys, values), **TOL)
 
 
-def test_prefill_f32_strided_rows_and_moving_reference(device) -> None:
+@pytest.mark.parametrize(("hq", "hkv"), [(8, 2), (32, 4)])
+def test_prefill_f32_strided_rows_and_moving_reference(device, hq, hkv) -> None:
     """Query and output rows inside wider ones, and keys that grow along each sequence, so
-    that the softmax reference moves many times."""
+    that the softmax reference moves many times: few rows (on the VALU kernel) and more."""
 
-    batch = workloads.paged_batch([700, 40], [200, 40], num_q_heads=8, num_kv_heads=2,
+    batch = workloads.paged_batch([700, 40], [200, 40], num_q_heads=hq, num_kv_heads=hkv,
                                   head_dim=64, block_size=16, dtype=torch.float32, device=device,
                                   seed=3)
     for b, context in enumerate([700, 40]):
         for i in range((context + 15) // 16):
             batch.key_cache[0, int(batch.block_tables[b, i])] *= 1 + i / 8
-    wide = torch.zeros(240, 8, 72, device=device)
+    wide = torch.zeros(240, hq, 72, device=device)
     wide[..., :64] = batch.query
-    out = torch.full((240, 12, 64), 7.0, device=device)
+    out = torch.full((240, hq + 4, 64), 7.0, device=device)
     ops.paged_attention_prefill(
         wide[..., :64], batch.key_cache, batch.value_cache, batch.block_tables, batch.seq_lens,
-        batch.cu_seqlens_q, layer_index=0, max_query_len=200, max_seq_len=700, out=out[:, :8])
+        batch.cu_seqlens_q, layer_index=0, max_query_len=200, max_seq_len=700, out=out[:, :hq])
     torch.cuda.synchronize()
     expected = _oracle(batch, batch.key_cache.cpu(), batch.value_cache.cpu())
     # Scores reach ~30 here, where one fp32 rounding is up to 2^-20; a sum of Dh products
     # gathers about sqrt(Dh) = 8 of them, so an exponent is off by up to 8e-6 and an output
     # by twice that times the largest |v| (~4).
-    assert_close(out[:, :8].cpu(), expected, rtol=0, atol=6e-5)
-    assert bool((out[:, 8:] == 7.0).all())
+    assert_close(out[:, :hq].cpu(), expected, rtol=0, atol=6e-5)
+    assert bool((out[:, hq:] == 7.0).all())
 
 
 @pytest.mark.parametrize("dh", [64, 128])
@@ -104,14 +105,20 @@ def test_prefill_f32_values_past_a_row_do_not_reach_it(device, dh, bad) -> None:
 
 
 @pytest.mark.parametrize("pool", ["same", "fp8_rows"])
-@pytest.mark.parametrize(("contexts", "chunks"),
-                         [([496, 90], [20, 28]), ([512, 90], [20, 28]), ([600, 90], [20, 29])])
-def test_prefill_f32_few_rows_over_many_keys(device, contexts, chunks, pool) -> None:
-    """Both sides of the rule that leaves few rows over many keys to the VALU kernel: below 512
-    keys and from there on, 48 and 49 tokens of 32 heads x 128."""
+@pytest.mark.parametrize(("contexts", "chunks", "layer"), [
+    ([496, 90], [20, 28], (32, 8, 128)), ([512, 90], [20, 28], (32, 8, 128)),
+    ([600, 90], [20, 29], (32, 8, 128)), ([112, 90], [9, 11], (32, 8, 128)),
+    ([128, 90], [9, 11], (32, 8, 128)), ([128, 90], [10, 11], (32, 8, 128)),
+    ([4000, 90], [60, 44], (32, 4, 64)), ([4000, 90], [60, 45], (32, 4, 64)),
+    ([3980, 90], [60, 44], (32, 4, 64))])
+def test_prefill_f32_few_rows_over_many_keys(device, contexts, chunks, layer, pool) -> None:
+    """Both sides of the rules that leave few rows over many keys to the VALU kernel: 48 and 49
+    tokens of 32 heads x 128 below and from 512 keys, 20 and 21 from 128 (fp32 pools), 104 and
+    105 of 32 heads x 64 from 4,000."""
 
     kw = dict(kv_dtype=torch.float8_e4m3fn, scale_granularity="row") if pool != "same" else {}
-    batch = workloads.paged_batch(contexts, chunks, num_q_heads=32, num_kv_heads=8, head_dim=128,
+    hq, hkv, dh = layer
+    batch = workloads.paged_batch(contexts, chunks, num_q_heads=hq, num_kv_heads=hkv, head_dim=dh,
                                   block_size=16, dtype=torch.float32, device=device, seed=6, **kw)
     got = _run(batch, batch.key_cache, batch.value_cache, **batch.scale_kwargs)
     pools = []

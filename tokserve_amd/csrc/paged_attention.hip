@@ -429,6 +429,10 @@ constexpr int64_t kSplitKeysFp8 = 1280;
 constexpr int64_t kSplitItemsFp8 = 448;
 constexpr int64_t kFewElements = int64_t{3} << 16;  // fp32 prefill: see prefill_impl
 constexpr int32_t kFewKeys = 512;
+constexpr int64_t kFewestElements = int64_t{5} << 14;
+constexpr int32_t kFewestKeys = 128;
+constexpr int64_t kFewLongElements = int64_t{13} << 14;
+constexpr int32_t kFewLongKeys = 4000;
 constexpr int32_t kWideKeys = 640;  // fp32: see decode_impl
 constexpr int32_t kWideKeys128 = 384;
 
@@ -835,9 +839,21 @@ int32_t prefill_impl(const void *query, int64_t q_token_stride, int64_t q_head_s
   // 8 / 2, Dh 64, 200 tokens: 139 and 226 us at 4,000; 512 in eight: 273 and 220 us. (Over
   // e4m3 pools at Dh 128 the VALU kernel reads V a byte at a time: 555 and 384 us for the
   // four chunks, so only up to 16 of its workgroups go there: one token, 347 and 361 us.)
-  const bool few = num_tokens * num_kv_heads <= 2 * kFillItems &&
-                   num_tokens * num_q_heads * head_dim <= kFewElements && key_cap >= kFewKeys &&
-                   (!fp8_pools || head_dim <= 64 || num_tokens * num_kv_heads <= 16);
+  // Two more corners: very few rows over fp32 pools from kFewestKeys keys (8 / 2, Dh 64, 48
+  // tokens in three chunks at 300: 15 and 20 us; 32 / 4 in eight of 3 is the worst, 1.19 of
+  // the other's time), and at Dh 64 up to four workgroups per CU over very many keys (32 / 4,
+  // 100 tokens at 8,100: 348 and 429 us; 8 / 2, 400 in eight at 4,060 1.19 of the other's).
+  // Over 2,376 batches of up to 1,000 tokens and 9,000 keys 32 are more than 5 % slower than
+  // on the VALU kernel (at most 24 %), the mean takes 0.45 of its time.
+  const int64_t workgroups = num_tokens * num_kv_heads;
+  const int64_t elements = num_tokens * num_q_heads * head_dim;
+  const bool few =
+      (workgroups <= 2 * kFillItems && elements <= kFewElements && key_cap >= kFewKeys &&
+       (!fp8_pools || head_dim <= 64 || workgroups <= 16)) ||
+      (workgroups <= 2 * kFillItems && elements <= kFewestElements && key_cap >= kFewestKeys &&
+       !fp8_pools) ||
+      (workgroups <= 4 * kFillItems && elements <= kFewLongElements && key_cap >= kFewLongKeys &&
+       head_dim <= 64);
   if (dtype == TKS_FLOAT32 && !few && scale_log2 > 0.f && scale_log2 < INFINITY &&
       prefill_f32_supported(head_dim, G, num_seqs, num_tokens, num_kv_heads, max_query_len) &&
       aligned16(query) && aligned16(out) &&
