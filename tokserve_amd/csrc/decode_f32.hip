@@ -14,7 +14,7 @@
 // Against the VALU kernel: 128 sequences of up to 8,192 keys (32 / 8 heads, Dh 128) 1,214
 // -> 387 us (5.1 TB/s), 128 of up to 1,152 (32 / 4, Dh 64, RoPE and append included) 93 ->
 // 38 us, 33 over e4m3 pools with row scales 730 -> 60 us, the small step (8 sequences of up
-// to 513 keys, 8 / 2, Dh 64, three launches before) 27 -> 21 us.
+// to 513 keys, 8 / 2, Dh 64, three launches before) 27 -> 12.6 us.
 //
 // ROPE: RoPE and the KV append of the new tokens in the same launch, as in decode_pv.hpp:
 // the query is rotated while it is staged, and the wave with the sequence's last page

@@ -4,7 +4,7 @@
 // Bound: the fp32 MFMA rate, 256 flop per CU and cycle (157 TFLOP/s at 2.4 GHz, a 16th of
 // bf16's), and the VALU beside it (one does not hide the other: a step's 64 MFMAs take
 // 2,048 cycles of a SIMD, its about 130 VALU instructions some 600). 16 prompts of 64 to
-// 1,024 tokens (32 / 4 heads, Dh 64): 828 us on the VALU kernel, 124 us here (87 TFLOP/s
+// 1,024 tokens (32 / 4 heads, Dh 64): 828 us on the VALU kernel, 117 us here (92 TFLOP/s
 // of visible scores). One workgroup of 4 waves per (sequence, KV head, 64 rows), row =
 // query token * G + query head, 16 rows a wave. Two 16-row tiles a wave halve the loads
 // but also the workgroups, and the longest of them then set the time: 152 us.
@@ -29,8 +29,7 @@ namespace {
 
 constexpr int kFWaves = 4;
 constexpr int kFKeys = 32;  // keys per step
-constexpr int kFTiles = 1;  // 16-row tiles per wave
-constexpr int kFRows = kFWaves * kFTiles * 16;
+constexpr int kFRows = kFWaves * 16;
 
 // This thread's part of one K (or V) row of a step, as loaded: DH / 8 elements.
 template <typename KV, int DH>
@@ -151,7 +150,6 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
   __shared__ __attribute__((aligned(16))) float ks_s[2][ROWS ? kFKeys : 4];
   __shared__ __attribute__((aligned(16))) float vs_s[2][ROWS ? kFKeys : 4];
 
-
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -237,37 +235,24 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
   };
   load_rows(0);  // (a step past the last loads nothing)
 
-  // Q^T operands of row tile j: rows (wave * kFTiles + j) * 16 + r. qpos: the last key the
-  // row sees (-1: none, or a padding row).
-  f32x4 qf[kFTiles][QC];
-  int qpos[kFTiles];
-  int min_pos = 0x7fffffff;
+  // Q^T operands of row wave * 16 + r. qpos: the last key it sees (-1: none, or padding).
+  const int row = wave * 16 + r;
+  const int token = t0 + row / G, head = kvh * G + row % G;
+  const bool in = row < QT * G && token < t_end;
+  const int qpos = in ? max(-1, min(base_pos + token, a.key_cap - 1)) : -1;
+  const int min_pos = __reduce_min_sync(~0ull, in ? qpos : 0x7fffffff);
+  const float *qp = q + (int64_t)(q0 + min(token, q_len - 1)) * a.q_ts + (int64_t)head * a.q_hs;
+  f32x4 qf[QC];
 #pragma unroll
-  for (int j = 0; j < kFTiles; ++j) {
-    const int row = (wave * kFTiles + j) * 16 + r;
-    const int t = t0 + row / G, h = row % G;
-    const bool in = row < QT * G && t < t_end;
-    qpos[j] = in ? max(-1, min(base_pos + t, a.key_cap - 1)) : -1;
-    min_pos = in ? min(min_pos, qpos[j]) : min_pos;
-    const float *qp = q + (int64_t)(q0 + min(t, q_len - 1)) * a.q_ts + (int64_t)(kvh * G + h) * a.q_hs;
-#pragma unroll
-    for (int c = 0; c < QC; ++c)
-      qf[j][c] = in ? *reinterpret_cast<const f32x4 *>(qp + 16 * c + 4 * g)
-                    : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  min_pos = __reduce_min_sync(~0ull, min_pos);
+  for (int c = 0; c < QC; ++c)
+    qf[c] = in ? *reinterpret_cast<const f32x4 *>(qp + 16 * c + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
 
-  f32x4 acc[kFTiles][4 * VC];
-  // Online softmax of tile j's row r, in log2 units: m the reference maximum (it moves
-  // when a score passes it by more than 8), l this lane's share of the sum.
-  float m[kFTiles], l[kFTiles];
+  f32x4 acc[4 * VC];
+  // Online softmax of row r, in log2 units: m the reference maximum (it moves when a score
+  // passes it by more than 8), l this lane's share of the sum.
+  float m = -INFINITY, l = 0.f;
 #pragma unroll
-  for (int j = 0; j < kFTiles; ++j) {
-    m[j] = -INFINITY;
-    l[j] = 0.f;
-#pragma unroll
-    for (int d = 0; d < 4 * VC; ++d) acc[j][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int d = 0; d < 4 * VC; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   const float scale_log2 = a.scale_log2;  // > 0 (the host routes other scales elsewhere)
 
   store_rows(Slot<0>{});
@@ -278,7 +263,7 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
     load_rows(s + 1);
     const int k0 = s * kFKeys;
 
-    f32x4 st[kFTiles][2] = {};
+    f32x4 st[2] = {};
 #pragma unroll
     for (int c = 0; c < QC; ++c) {
       f32x4 kf[2];
@@ -288,9 +273,7 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int j = 0; j < kFTiles; ++j) st[j][kt] = mfma_f32(kf[kt][e], qf[j][c][e], st[j][kt]);
+        for (int kt = 0; kt < 2; ++kt) st[kt] = mfma_f32(kf[kt][e], qf[c][e], st[kt]);
     }
     f32x4 vs4[2];
     if constexpr (ROWS) {
@@ -298,8 +281,7 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
       for (int kt = 0; kt < 2; ++kt) {
         const f32x4 ks4 = *reinterpret_cast<const f32x4 *>(&ks_s[buf][kt * 16 + 4 * g]);
         vs4[kt] = *reinterpret_cast<const f32x4 *>(&vs_s[buf][kt * 16 + 4 * g]);
-#pragma unroll
-        for (int j = 0; j < kFTiles; ++j) st[j][kt] *= ks4;
+        st[kt] *= ks4;
       }
     }
     // Steps past the wave's first query position: key k0 + kt*16 + 4g + i is seen iff it
@@ -307,41 +289,36 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
     const bool need_mask = k0 + kFKeys - 1 > min_pos;
     if (need_mask) {
 #pragma unroll
-      for (int j = 0; j < kFTiles; ++j)
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (k0 + kt * 16 + 4 * g + i > qpos[j]) st[j][kt][i] = -INFINITY;
-    }
-#pragma unroll
-    for (int j = 0; j < kFTiles; ++j) {
-      const float a0 = nan_max(nan_max(st[j][0][0], st[j][0][1]), nan_max(st[j][0][2], st[j][0][3]));
-      const float a1 = nan_max(nan_max(st[j][1][0], st[j][1][1]), nan_max(st[j][1][2], st[j][1][3]));
-      const float lm = nan_max(a0, a1) * scale_log2;
-      if (__builtin_amdgcn_ballot_w64(lm > m[j] + 8.f)) {
-        const float mx = xgroup_max(lm);
-        const bool bump = mx > m[j] + 8.f;
-        const float alpha = bump ? fast_exp2(m[j] - mx) : 1.f;
-        m[j] = bump ? mx : m[j];
-        l[j] *= alpha;
-#pragma unroll
-        for (int d = 0; d < 4 * VC; ++d) acc[j][d] *= alpha;
-      }
-      const float nr = m[j] == -INFINITY ? 0.f : -m[j];
-      float sum[2];
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
+      for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          st[j][kt][i] = fast_exp2(__builtin_fmaf(st[j][kt][i], scale_log2, nr));
-        sum[kt] = (st[j][kt][0] + st[j][kt][1]) + (st[j][kt][2] + st[j][kt][3]);
-      }
-      l[j] += sum[0] + sum[1];
-      if constexpr (ROWS) {
+          if (k0 + kt * 16 + 4 * g + i > qpos) st[kt][i] = -INFINITY;
+    }
+    const float a0 = nan_max(nan_max(st[0][0], st[0][1]), nan_max(st[0][2], st[0][3]));
+    const float a1 = nan_max(nan_max(st[1][0], st[1][1]), nan_max(st[1][2], st[1][3]));
+    const float lm = nan_max(a0, a1) * scale_log2;
+    if (__builtin_amdgcn_ballot_w64(lm > m + 8.f)) {
+      const float mx = xgroup_max(lm);
+      const bool bump = mx > m + 8.f;
+      const float alpha = bump ? fast_exp2(m - mx) : 1.f;
+      m = bump ? mx : m;
+      l *= alpha;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) st[j][kt] *= vs4[kt];
-      }
+      for (int d = 0; d < 4 * VC; ++d) acc[d] *= alpha;
+    }
+    const float nr = m == -INFINITY ? 0.f : -m;
+    float sum[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        st[kt][i] = fast_exp2(__builtin_fmaf(st[kt][i], scale_log2, nr));
+      sum[kt] = (st[kt][0] + st[kt][1]) + (st[kt][2] + st[kt][3]);
+    }
+    l += sum[0] + sum[1];
+    if constexpr (ROWS) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) st[kt] *= vs4[kt];
     }
 
     auto v_operand = [&](int kt, int i, int h) {
@@ -352,24 +329,19 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
     // 2.1e-7, 2.5e-7 with one; the VALU kernel's is 2.3e-7).
 #pragma unroll
     for (int h = 0; h < VC; ++h) {
-      f32x4 o[kFTiles][4] = {};
+      f32x4 o[4] = {};
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float4 vf = v_operand(kt, i, h);
-#pragma unroll
-          for (int j = 0; j < kFTiles; ++j) {
-            o[j][0] = mfma_f32(vf.x, st[j][kt][i], o[j][0]);
-            o[j][1] = mfma_f32(vf.y, st[j][kt][i], o[j][1]);
-            o[j][2] = mfma_f32(vf.z, st[j][kt][i], o[j][2]);
-            o[j][3] = mfma_f32(vf.w, st[j][kt][i], o[j][3]);
-          }
+          o[0] = mfma_f32(vf.x, st[kt][i], o[0]);
+          o[1] = mfma_f32(vf.y, st[kt][i], o[1]);
+          o[2] = mfma_f32(vf.z, st[kt][i], o[2]);
+          o[3] = mfma_f32(vf.w, st[kt][i], o[3]);
         }
 #pragma unroll
-      for (int j = 0; j < kFTiles; ++j)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) acc[j][4 * h + d] += o[j][d];
+      for (int d = 0; d < 4; ++d) acc[4 * h + d] += o[d];
       register_fence<DH>();
     }
     store_rows(Slot<buf ^ 1>{});
@@ -385,18 +357,15 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
   // finite takes its rows one by one.
   float bad = 0.f;
 #pragma unroll
-  for (int j = 0; j < kFTiles; ++j)
+  for (int d = 0; d < 4 * VC; ++d)
 #pragma unroll
-    for (int d = 0; d < 4 * VC; ++d)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bad += 0.f * acc[j][d][i];
+    for (int i = 0; i < 4; ++i) bad += 0.f * acc[d][i];
   if (__builtin_amdgcn_ballot_w64(bad != bad)) {
 #pragma unroll 1
-    for (int k = 0; k < kFTiles * 16; ++k) {
-      const int row = wave * kFTiles * 16 + k;
-      const int t = t0 + row / G, h = row % G;
-      if (row < QT * G && t < t_end)
-        one_row<KV, DH>(a, kvh * G + h, kc, vc, head_base, bt_row, q0 + t,
+    for (int k = 0; k < 16; ++k) {
+      const int x = wave * 16 + k, t = t0 + x / G;
+      if (x < QT * G && t < t_end)
+        one_row<KV, DH>(a, kvh * G + x % G, kc, vc, head_base, bt_row, q0 + t,
                         max(0, min(base_pos + t + 1, a.key_cap)), lane);
     }
     return;
@@ -404,24 +373,19 @@ void prefill_f32_kernel(PrefillArgs a, int G) {
 
   // Lane (g, r) holds dims 64 h + 16 g + 4 i + d of row r in acc[4 h + d][i].
   float *out = static_cast<float *>(a.out);
+  l = xgroup_sum(l);
+  if (!in) return;
+  const bool any = qpos >= 0;  // a row without keys is zero
+  float *op = out + (int64_t)(q0 + token) * a.o_ts + (int64_t)head * a.o_hs + 16 * g;
 #pragma unroll
-  for (int j = 0; j < kFTiles; ++j) {
-    const float lj = xgroup_sum(l[j]);
-    const int row = (wave * kFTiles + j) * 16 + r;
-    const int t = t0 + row / G, h = row % G;
-    if (row >= QT * G || t >= t_end) continue;
-    const bool any = qpos[j] >= 0;  // a row without keys is zero
-    float *op = out + (int64_t)(q0 + t) * a.o_ts + (int64_t)(kvh * G + h) * a.o_hs + 16 * g;
+  for (int c = 0; c < VC; ++c)
 #pragma unroll
-    for (int c = 0; c < VC; ++c)
+    for (int i = 0; i < 4; ++i) {
+      float o[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float o[4];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) o[d] = any ? acc[j][4 * c + d][i] / lj * a.v_scale : 0.f;
-        *reinterpret_cast<float4 *>(op + 64 * c + 4 * i) = make_float4(o[0], o[1], o[2], o[3]);
-      }
-  }
+      for (int d = 0; d < 4; ++d) o[d] = any ? acc[4 * c + d][i] / l * a.v_scale : 0.f;
+      *reinterpret_cast<float4 *>(op + 64 * c + 4 * i) = make_float4(o[0], o[1], o[2], o[3]);
+    }
 }
 
 template <typename KV, bool ROWS>

@@ -4,7 +4,7 @@
 // operators' device kernels). Small calls last as long as the host takes for them: the
 // fused decode of 8 sequences 20.6 us through the ctypes binding and 12.5 us from here, the
 // greedy choice of 16 rows 10.6 and 6.8 us, a 1.1B model's iteration (about 200 calls)
-// 5,060 and 4,270 us.
+// 5,060 and 4,000 us.
 //
 // The entry points are looked up in libtokserve_hip.so on the first call, so loading this
 // library does not touch HIP. It is loaded and registered by torch_ops.py, which first
