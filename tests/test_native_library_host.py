@@ -51,6 +51,19 @@ def test_a_library_of_other_versions_is_not_registered(tmp_path, torch_version, 
     assert message in error and "registered" not in error
 
 
+@pytest.mark.parametrize("version", ["2.10.0", "2.10.0+rocm7.0", "2.10.0a0+git1234",
+                                     "2.10.0.dev20250101"])
+def test_builds_of_one_release_fit(tmp_path, monkeypatch, version) -> None:
+    (tmp_path / "stub.c").write_text(
+        'const char *tks_torch_built_for(void) { return "2.10.0"; }\n'
+        f"int tks_torch_abi_version(void) {{ return {_lib.ABI_VERSION}; }}\n"
+        'const char *tks_torch_register(void) { return 0; }\n')
+    stub = tmp_path / "stub.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", stub, tmp_path / "stub.c"], check=True)
+    monkeypatch.setattr(torch, "__version__", version)
+    assert torch_ops._load_native(stub) is None
+
+
 def test_make_without_a_torch_builds_the_c_library_alone() -> None:
     run = subprocess.run(["make", "-n", "-C", CSRC, "PYTHON=false"], capture_output=True, text=True)
     assert run.returncode == 0, run.stderr

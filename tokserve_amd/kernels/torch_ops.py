@@ -37,6 +37,7 @@ kernels are Triton functions behind tokserve/kernels/<op>.py):
 from __future__ import annotations
 
 import ctypes
+import re
 from pathlib import Path
 
 import torch
@@ -310,7 +311,8 @@ def _load_native(path: Path) -> str | None:
         abi_version = library.tks_torch_abi_version()
     except (OSError, AttributeError) as error:
         return f"{path} does not load into torch {torch.__version__} ({error}){rebuild}"
-    if torch_version != torch.__version__.split("+")[0]:
+    # (the macro holds the release alone: 2.10.0 also of 2.10.0a0+git and 2.10.0+rocm7.0)
+    if torch_version != re.match(r"\d+(\.\d+)*", torch.__version__).group():
         return (f"{path} was built for torch {torch_version}, not {torch.__version__}"
                 f"{rebuild}")
     if abi_version != _lib.ABI_VERSION:
